@@ -241,6 +241,15 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + PW) * OCC + 3) / 4))) void gemm_t
   constexpr bool kResLds = PW > 0 && !STREAMK && epi_has_resid<epi_base(EPI)>() &&
                            (S::kLdsBytes + BM * BN * 2) * OCC <= 160 * 1024 && (BM * BN * 2 / 1024) % PW == 0;
   constexpr int kResBytes = kResLds ? BM * BN * 2 : 0;
+  // Row statistics of a fused pre-norm: under stream-K each compute wave sums
+  // the rows it multiplies (RowSums); the tile kernels read those of a pass
+  // before them.  They were built with sums of their own, both ways, and lost
+  // what the pass costs: in the producer waves, from the landed stages, the
+  // sums delayed the refills (ModernBERT-base Wi+LN at 8109 tokens 48.9 us
+  // against 49.3 with the pass, Qwen3.5-small in_proj at 8192 409.6 against
+  // 378.5); in the compute waves they spilled (58.0 and 459.4 us).
+  constexpr bool kStatPass = !STREAMK || epi_base(EPI) == kEpiConvSilu;
+  constexpr int kOwnNorm = kStatPass ? kNormNone : epi_norm(EPI);
   __shared__ __attribute__((aligned(1024))) char lds[S::kLdsBytes + kResBytes];
   char* const res_lds = lds + S::kLdsBytes;
   // (every k-tile loop needs two k-steps per tile, so that a tile's copy,
@@ -478,8 +487,14 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + PW) * OCC + 3) / 4))) void gemm_t
       f.w[i] = *reinterpret_cast<const i32x4*>(base + wrow_off[i] + ((c ^ wrow_swz[i]) << 4));
   };
 
+  // Row sums taken by the compute waves: lane l holds row l % 32 of each x
+  // block over the k-chunks of its half (l / 32).  Every wave sums the rows
+  // it multiplies, so nothing is exchanged between waves.
+  RowSums<kOwnNorm> sums[S::FM];
   f32x16 acc[S::FN][S::FM];
   auto zero_acc = [&]() {
+#pragma unroll
+    for (int j = 0; j < S::FM; ++j) sums[j] = RowSums<kOwnNorm>();
 #pragma unroll
     for (int i = 0; i < S::FN; ++i)
 #pragma unroll
@@ -493,7 +508,10 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + PW) * OCC + 3) / 4))) void gemm_t
 #pragma unroll
     for (int i = 0; i < S::FN; ++i)
 #pragma unroll
-      for (int j = 0; j < S::FM; ++j) acc[i][j] = mfma32(f.w[i], f.x[j], acc[i][j]);
+      for (int j = 0; j < S::FM; ++j) {
+        acc[i][j] = mfma32(f.w[i], f.x[j], acc[i][j]);
+        if (i == 0) sums[j].add(f.x[j]);
+      }
   };
   // The same MFMAs with DMA instructions [I0, I0 + N) of refill `r` spread
   // evenly between them (after MFMA q go instructions I0 + q*N/Q ..
@@ -508,6 +526,7 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + PW) * OCC + 3) / 4))) void gemm_t
       for (int j = 0; j < S::FM; ++j) {
         const int q = i * S::FM + j;
         acc[i][j] = mfma32(f.w[i], f.x[j], acc[i][j]);
+        if (i == 0) sums[j].add(f.x[j]);
 #pragma unroll
         for (int d = I0 + q * N / Q; d < I0 + (q + 1) * N / Q; ++d) dma_one(r, d);
         __builtin_amdgcn_sched_barrier(0);
@@ -536,15 +555,27 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + PW) * OCC + 3) / 4))) void gemm_t
   // into w, c_n = sum_k of folded row n); then the base epilogue E runs.
   constexpr int E = epi_base(EPI);
   constexpr int NORM = epi_norm(EPI);
-  // A tile's row statistics and column sums are all loaded before any of
-  // them is used, so the epilogue waits for one round trip, not one per
-  // block.
+  // (A tile's column sums, and the statistics of a pass before, are all
+  // loaded before any of them is used, so the epilogue waits for one round
+  // trip, not one per block.)
   auto normalize_tile = [&](int m0, int n0) {
-    float rs[S::FM];
+    float mu[S::FM], rs[S::FM];
 #pragma unroll
     for (int j = 0; j < S::FM; ++j) {
-      const int m = min(m0 + wm * S::TM + j * 32 + frow, a.M - 1);
-      rs[j] = a.stats[2 * (int64_t)m + 1];
+      const int row0 = m0 + wm * S::TM + j * 32;
+      if constexpr (kStatPass) {
+        const int m = min(row0 + frow, a.M - 1);
+        mu[j] = a.stats[2 * (int64_t)m];
+        rs[j] = a.stats[2 * (int64_t)m + 1];
+      } else {
+        // both halves of the row's k-chunks
+        const float s = sums[j].s + __shfl_xor(sums[j].s, 32, 64), q = sums[j].q + __shfl_xor(sums[j].q, 32, 64);
+        float var;
+        const bool bad = row_stats_from_sums<kOwnNorm>(s, q, a.K, mu[j], var);
+        if constexpr (kOwnNorm == kNormLayer)
+          exact_row_stats(__ballot(bad) & 0xffffffffull, a.x, a.ldx, row0, a.M - 1, a.K, lane, 31, mu[j], var);
+        rs[j] = 1.0f / sqrtf(var + a.eps);
+      }
     }
     if constexpr (NORM == kNormLayer) {
       // acc - mu_m c_n as one more MFMA per block: A holds c_n's bf16 split
@@ -564,8 +595,7 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + PW) * OCC + 3) / 4))) void gemm_t
       }
 #pragma unroll
       for (int j = 0; j < S::FM; ++j) {
-        const int m = min(m0 + wm * S::TM + j * 32 + frow, a.M - 1);
-        const float nm = -a.stats[2 * (int64_t)m];
+        const float nm = -mu[j];
         const __bf16 hi = to_bf16(nm), lo = to_bf16(nm - to_f32(hi));
         bf16x8 v = {};
         if (fk == 0) v[0] = hi, v[1] = lo, v[2] = hi;
@@ -892,6 +922,12 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + PW) * OCC + 3) / 4))) void gemm_t
   auto slot_off = [&](int g, int slot) -> unsigned {  // byte offset of this lane's first f32x4
     return (unsigned)((((int64_t)g * 2 + slot) * kTileF4 + wave * kWaveF4 + lane) * 16);
   };
+  // The row sums of a fused pre-norm go the same way, to a.stats:
+  // [workgroup][slot][wave][block j][64 lanes] of (sum, sum of squares).
+  const rsrc_t ssr = make_rsrc(a.stats);
+  auto sums_off = [&](int g, int slot) -> unsigned {
+    return (unsigned)(((((int64_t)g * 2 + slot) * S::kWaves + wave) * S::FM * 64 + lane) * 8);
+  };
   // A partial segment: write this workgroup's partial; returns true when it
   // is the tile's last segment to arrive, with acc then holding the full sum
   // (the caller runs the epilogue).
@@ -916,6 +952,13 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + PW) * OCC + 3) / 4))) void gemm_t
         }
         __builtin_amdgcn_sched_barrier(0);
       }
+    if constexpr (kOwnNorm != kNormNone) {
+#pragma unroll
+      for (int j = 0; j < S::FM; ++j)
+        __builtin_amdgcn_raw_buffer_store_b64(
+            (i32x2){__builtin_bit_cast(int, sums[j].s), __builtin_bit_cast(int, sums[j].q)}, ssr,
+            (int)(sums_off(blockIdx.x, slot) + j * 64 * 8), 0, kCoherent);
+    }
     int g_lo, g_hi;
     walk.tile_owners(t, g_lo, g_hi);
     // Each wave arrives on its own counter (tile, wave): its slice of the
@@ -933,7 +976,18 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + PW) * OCC + 3) / 4))) void gemm_t
     const int64_t tile_lo = (int64_t)t * walk.kt_count;
     for (int g = g_lo; g <= g_hi; ++g) {
       // g's segment in this tile is its head iff g's range starts inside the tile.
-      const unsigned src = slot_off(g, walk.start(g) >= tile_lo ? 0 : 1);
+      const int gslot = walk.start(g) >= tile_lo ? 0 : 1;
+      const unsigned src = slot_off(g, gslot);
+      if constexpr (kOwnNorm != kNormNone) {
+#pragma unroll
+        for (int j = 0; j < S::FM; ++j) {
+          typedef float f32x2_t __attribute__((ext_vector_type(2)));
+          const f32x2_t v = __builtin_bit_cast(
+              f32x2_t, __builtin_amdgcn_raw_buffer_load_b64(ssr, (int)(sums_off(g, gslot) + j * 64 * 8), 0, kCoherent));
+          sums[j].s += v[0];
+          sums[j].q += v[1];
+        }
+      }
       // All of one owner's loads are in flight together (these coherent
       // reads come from beyond the L2: one round trip per owner, not one
       // per block), then added in the same order as always.

@@ -20,13 +20,6 @@
 
 namespace sys1 {
 
-// Sum over the 64 lanes of a wave, the same order on every call.
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
-}
-
 // One wave per row: stats[2m] = mean (0 for RMSNorm), stats[2m+1] =
 // 1/sqrt(var + eps).  LayerNorm takes the variance about the mean, as the
 // reference does: the row is loaded once into registers (all its loads in

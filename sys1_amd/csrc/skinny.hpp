@@ -109,28 +109,22 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs a) {
       if constexpr (kBiasPre) bias_pre = load8_bf16(a.bias + n, a.Nout - n);
     }
   }
-  // The pre-norm epilogues' row statistics and column sums (written by
-  // the statistics pass before this launch), likewise.
-  constexpr bool kNormPre = NORM != kNormNone && kOnePerThread;
-  float rs_pre = 0.0f, mu_pre = 0.0f, cs_pre[kNormPre && NORM == kNormLayer ? 8 : 1] = {};
-  if constexpr (kNormPre) {
-    const int t = threadIdx.x;
-    const int m = min(m0 + t / kVecs, a.M - 1), c0 = (t % kVecs) * 8;
-    rs_pre = a.stats[2 * (int64_t)m + 1];
-    if constexpr (NORM == kNormLayer) {
-      mu_pre = a.stats[2 * (int64_t)m];
-      if (n0 + c0 + 8 <= a.N) {  // two 16-byte reads (kNormPre implies not gated)
-        const f32x4 c0v = *reinterpret_cast<const f32x4*>(a.colsum + n0 + c0);
-        const f32x4 c1v = *reinterpret_cast<const f32x4*>(a.colsum + n0 + c0 + 4);
+  // LayerNorm's column sums likewise.
+  constexpr bool kColPre = NORM == kNormLayer && kOnePerThread;
+  float cs_pre[kColPre ? 8 : 1] = {};
+  if constexpr (kColPre) {
+    const int c0 = ((int)threadIdx.x % kVecs) * 8;
+    if (n0 + c0 + 8 <= a.N) {  // two 16-byte reads (kColPre implies not gated)
+      const f32x4 c0v = *reinterpret_cast<const f32x4*>(a.colsum + n0 + c0);
+      const f32x4 c1v = *reinterpret_cast<const f32x4*>(a.colsum + n0 + c0 + 4);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          cs_pre[e] = c0v[e];
-          cs_pre[4 + e] = c1v[e];
-        }
-      } else {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) cs_pre[e] = a.colsum[min(n0 + c0 + e, a.N - 1)];
+      for (int e = 0; e < 4; ++e) {
+        cs_pre[e] = c0v[e];
+        cs_pre[4 + e] = c1v[e];
       }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) cs_pre[e] = a.colsum[min(n0 + c0 + e, a.N - 1)];
     }
   }
 
@@ -154,13 +148,19 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs a) {
         bx[b][u][j] = __builtin_amdgcn_raw_buffer_load_b128(xr, ok ? (int)xo[j] : (int)kOutOfRange, so, 0);
     }
   };
+  // Row sums of a fused pre-norm, over this lane's k-chunks of its rows
+  // (chunks past K and k-steps past the range are zeros).
+  RowSums<NORM> sums[FM];
   auto compute = [&](int b) {
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int i = 0; i < FN; ++i)
 #pragma unroll
-        for (int j = 0; j < FM; ++j) acc[i][j] = mfma16(bw[b][u][i], bx[b][u][j], acc[i][j]);
+        for (int j = 0; j < FM; ++j) {
+          acc[i][j] = mfma16(bw[b][u][i], bx[b][u][j], acc[i][j]);
+          if (i == 0) sums[j].add(bx[b][u][j]);
+        }
   };
   if (s0 < s1) {
     load(0, s0);
@@ -182,7 +182,44 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs a) {
 #pragma unroll
     for (int j = 0; j < FM; ++j)
       *reinterpret_cast<f32x4*>(mine + (j * 16 + r16) * S::kRowF32 + i * 16 + 4 * q) = acc[i][j];
+  if constexpr (NORM != kNormNone) {
+    // ... and its row sums, over the four lanes of a row, to the two pad
+    // columns at BN.
+#pragma unroll
+    for (int j = 0; j < FM; ++j) {
+      float s = sums[j].s, qq = sums[j].q;
+      s += __shfl_xor(s, 16, 64);
+      qq += __shfl_xor(qq, 16, 64);
+      s += __shfl_xor(s, 32, 64);
+      qq += __shfl_xor(qq, 32, 64);
+      if (q == 0) {
+        mine[(j * 16 + r16) * S::kRowF32 + BN] = s;
+        mine[(j * 16 + r16) * S::kRowF32 + BN + 1] = qq;
+      }
+    }
+  }
   __syncthreads();
+  if constexpr (NORM != kNormNone) {
+    // The first BM threads finish a row's statistics each, into the other
+    // two pad columns of wave 0's slab.
+    if (wave * 64 < BM) {
+      const int r = min((int)threadIdx.x, BM - 1);
+      float s = 0.0f, qq = 0.0f, mean, var;
+#pragma unroll
+      for (int ww = 0; ww < NW; ++ww) {
+        s += red[(ww * BM + r) * S::kRowF32 + BN];
+        qq += red[(ww * BM + r) * S::kRowF32 + BN + 1];
+      }
+      const bool bad = row_stats_from_sums<NORM>(s, qq, a.K, mean, var) && (int)threadIdx.x < BM;
+      if constexpr (NORM == kNormLayer)
+        exact_row_stats(__ballot(bad), a.x, a.ldx, m0 + wave * 64, a.M - 1, a.K, lane, 63, mean, var);
+      if ((int)threadIdx.x < BM) {
+        red[r * S::kRowF32 + BN + 2] = mean;
+        red[r * S::kRowF32 + BN + 3] = 1.0f / sqrtf(var + a.eps);
+      }
+    }
+    __syncthreads();
+  }
 
   // Epilogue: each thread takes 8 consecutive output columns of one row,
   // sums the waves' partials in wave order, applies the epilogue in the
@@ -222,18 +259,17 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs a) {
     }
     // (for gated epilogues v holds the gate sums and g the up sums)
     if constexpr (NORM != kNormNone) {
-      const float r = kNormPre ? rs_pre : a.stats[2 * (int64_t)m + 1];
-      const float mu = NORM == kNormLayer ? (kNormPre ? mu_pre : a.stats[2 * (int64_t)m]) : 0.0f;
+      const float mu = red[r * S::kRowF32 + BN + 2], rs = red[r * S::kRowF32 + BN + 3];
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         if constexpr (NORM == kNormLayer) {
           const int wn = min(n0 + pc + e, a.N - 1);  // weight row of the gate (or plain) column
-          const float cs = kNormPre ? cs_pre[e] : a.colsum[wn];
-          v[e] = r * (v[e] - mu * cs);
-          if constexpr (kGated) g[e] = r * (g[e] - mu * a.colsum[min(wn + 16, a.N - 1)]);
+          const float cs = kColPre ? cs_pre[e] : a.colsum[wn];
+          v[e] = rs * (v[e] - mu * cs);
+          if constexpr (kGated) g[e] = rs * (g[e] - mu * a.colsum[min(wn + 16, a.N - 1)]);
         } else {
-          v[e] *= r;
-          if constexpr (kGated) g[e] *= r;
+          v[e] *= rs;
+          if constexpr (kGated) g[e] *= rs;
         }
       }
     }

@@ -83,7 +83,10 @@ struct Context {
   hipEvent_t order = nullptr;  // orders a new stream after the old one (sys1hip_set_stream)
   float* ws = nullptr;
   unsigned* counters = nullptr;
-  float* stats = nullptr;  // pre-norm row statistics, kNormRows x (mean, 1/std)
+  // Pre-norm row statistics of the pass, kNormRows x (mean, 1/std), or the
+  // partial row sums of a stream-K call: 8 bytes per row and wave column of
+  // each partial tile, at most 1/16 of the partials' bytes (4 MB of these 8).
+  float* stats = nullptr;
   // Projection chains: the dependency bank (zero between launches: each
   // launch's last workgroup clears it) and the error word, one allocation.
   unsigned* chain = nullptr;
@@ -166,6 +169,11 @@ int epi_id_from_flags(int32_t f) {
 }
 
 int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// Whether a pre-norm projection on kernel `e` reads the row statistics of a
+// pass in front of it (the tile kernels); the skinny and stream-K kernels
+// take them themselves.
+bool needs_stats_pass(const KernelEntry& e) { return !e.skinny && !e.streamk; }
 
 // Modelled time (in CU clocks) of a projection on kernel `e` launched on
 // `grid` workgroups, of which the first `dp` tiles run whole (tile phase)
@@ -1083,11 +1091,12 @@ int sys1hip_norm_linear_bf16(void* ctx, const uint16_t* x, int64_t ldx, const ui
   const KernelEntry& e = kKernels[p.kernel];
   if (e.streamk && (cdiv(M, e.bm) * cdiv(N, e.bn) - p.dp) * (e.threads / 64) > kCounterSlots)
     return fail(SYS1HIP_ERANGE, "sys1hip_norm_linear_bf16: more split tiles than stream-K counters");
-  const auto* xb = reinterpret_cast<const __bf16*>(x);
-  rc = launch_row_stats(c, xb, ldx, M, K, norm, eps);
-  if (rc) return rc;
+  if (needs_stats_pass(e)) {
+    rc = launch_row_stats(c, reinterpret_cast<const __bf16*>(x), ldx, M, K, norm, eps);
+    if (rc) return rc;
+  }
   GemmArgs a = {};
-  a.x = xb;
+  a.x = reinterpret_cast<const __bf16*>(x);
   a.w = reinterpret_cast<const __bf16*>(w_folded);
   a.y = reinterpret_cast<__bf16*>(y);
   a.ws = c->ws;
@@ -1098,6 +1107,7 @@ int sys1hip_norm_linear_bf16(void* ctx, const uint16_t* x, int64_t ldx, const ui
   a.group_m = raster_group(K);
   a.stats = c->stats;
   a.colsum = colsum;
+  a.eps = eps;
   a.w_kt = blocked ? (int)cdiv(K, kBlkK) : 0;
   hipLaunchKernelGGL(e.fn[epi], dim3((unsigned)p.grid), dim3(e.threads), 0, c->stream, a);
   HIP_TRY(hipGetLastError());
@@ -1164,7 +1174,8 @@ int sys1hip_linear_conv_silu_bf16(void* ctx, const uint16_t* x, int64_t ldx, con
   const int64_t rows = fused ? halo_rows(e, M, kConvHalo) : M;
   if (e.streamk && (cdiv(rows, e.bm) * cdiv(N, e.bn) - p.dp) * (e.threads / 64) > kCounterSlots)
     return fail(SYS1HIP_ERANGE, "sys1hip_linear_conv_silu_bf16: more split tiles than stream-K counters");
-  if (norm) {
+  a.eps = eps;
+  if (norm && (fused || needs_stats_pass(e))) {
     rc = launch_row_stats(c, xb, ldx, M, K, norm, eps);
     if (rc) return rc;
   }

@@ -227,3 +227,42 @@ def test_blocked_weight_with_every_norm_epilogue_is_bitwise_row_major(dev, orc):
                 assert_parity(to_np(b), ref, f"blocked {name} {kind}/{gated}")
     finally:
         dev.set_kernel(-1)
+
+
+@pytest.mark.parametrize("name,grid", [("skinny_16x16_w16", 0), ("skinny_128x32_w8", 0), ("skinny_64x48_w8", 0),
+                                       ("stream_32x256_s4_w1x4_p4", 7), ("stream_128x256_s3_w2x4", 5),
+                                       ("stream_64x256_s4_w2x4_p4", 3)])
+@pytest.mark.parametrize("kind", ["layer", "rms"])
+def test_row_sums_of_the_multiplying_kernels(dev, orc, name, grid, kind):
+    """The skinny and stream-K kernels take the row statistics from their own
+    fragments: rows on both sides of the mean^2 = 16 var line beyond which a
+    variance is taken about the mean (rows 6 and 16 deviations off zero, a
+    ragged last tile row, split tiles), and a row with an infinity, which
+    stays that row's alone.  Projection tolerance, as everywhere."""
+    from sys1_amd import kernel_names
+    from sys1_amd.norm import NormLinear
+    N, K = 330, 712
+    eps = 1e-5 if kind == "layer" else 1e-6
+    w, g = _weights(orc, N, K, 71, kind)
+    lin = NormLinear(to_gpu_bf16(w, torch), torch.from_numpy(g), kind, eps, None, device=dev)
+    try:
+        dev.set_kernel(kernel_names().index(name))
+        dev.set_grid(grid)
+        for M in (1, 17, 133):
+            print(f"[gpu] row sums {name} grid={grid} {kind} M={M}", flush=True)
+            x = orc.fill_normal((M, K), 80 + M)
+            x += np.array([0.0, 3.0, 6.0, -16.0, 0.1], np.float32)[np.arange(M) % 5][:, None]
+            x = orc.round_bf16(x)
+            ref = _ref(orc, x, w, g, kind, eps, None)
+            assert_parity(to_np(lin(to_gpu_bf16(x, torch))), ref, f"{name} {kind} M={M}")
+            if M == 1:
+                continue
+            x[7, 11] = np.inf
+            y = to_np(lin(to_gpu_bf16(x, torch)))
+            # LayerNorm: inf - inf; RMSNorm: inf / inf.  NaN throughout the row.
+            assert np.isnan(y[7]).all()
+            keep = np.arange(M) != 7
+            assert_parity(y[keep], ref[keep], f"{name} {kind} M={M} beside an infinity")
+    finally:
+        dev.set_kernel(-1)
+        dev.set_grid(0)
