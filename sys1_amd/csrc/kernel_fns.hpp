@@ -53,11 +53,12 @@ constexpr KernelFn conv_fn() {
 #ifdef SYS1_SKINNY_HPP
 namespace sys1 {
 // A skinny-M kernel per epilogue; null where the epilogue does not apply
-// (gated epilogues need whole 32-row gate/up groups, an even FN; RoPE and
-// conv run on the tile kernels).
+// (gated epilogues need whole 32-row gate/up groups, an even FN; RoPE half
+// or whole heads, FN = 2 or 4; the conv runs on the tile kernels).
 template <int FM, int FN, int NW, int U, int EPI>
 constexpr KernelFn skinny_fn() {
-  if constexpr ((epi_gated(EPI) && FN % 2 != 0) || epi_base(EPI) == kEpiRopeQkv || epi_base(EPI) == kEpiConvSilu)
+  if constexpr ((epi_gated(EPI) && FN % 2 != 0) || (EPI == kEpiRopeQkv && FN != 2 && FN != 4) ||
+                epi_base(EPI) == kEpiConvSilu)
     return nullptr;
   else
     return skinny_kernel<FM, FN, NW, U, EPI>;

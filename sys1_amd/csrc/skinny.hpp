@@ -24,6 +24,14 @@
 // Gated epilogues (GeGLU / SwiGLU) need an even FN: the packed gate/up
 // layout puts 16 gate rows and then the 16 matching up rows in each 32-row
 // group, i.e. in the workgroup's blocks 2g and 2g + 1.
+//
+// RoPE needs columns c and c + 32 of a 64-wide head in one workgroup, so FN
+// is 2 or 4 and the workgroup's second half of blocks is taken 32 columns
+// after its first: with FN = 2 two workgroups share a head (columns 0-15 |
+// 32-47 and 16-31 | 48-63), with FN = 4 a workgroup owns one.  The rotation
+// runs on the summed partials.  (Wqkv + RoPE ran on the tile and stream-K
+// kernels alone, whose waves own whole heads: ModernBERT-base at 61 tokens
+// 21.2 us on 15 x 3 stream-K ranges, against 6.9 us on 144 tiles here.)
 #pragma once
 #define SYS1_SKINNY_HPP
 
@@ -53,7 +61,9 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs a) {
   constexpr int NORM = epi_norm(EPI);
   constexpr bool kGated = epi_gated(E);
   static_assert(!kGated || FN % 2 == 0, "gated epilogues: whole 32-row gate/up groups per workgroup");
-  static_assert(E != kEpiRopeQkv && E != kEpiConvSilu, "RoPE and conv epilogues run on the tile kernels");
+  constexpr bool kRope = E == kEpiRopeQkv;
+  static_assert(!kRope || FN == 2 || FN == 4, "RoPE: half or whole heads per workgroup");
+  static_assert(E != kEpiConvSilu, "the conv epilogue runs on the tile kernels");
   __shared__ __attribute__((aligned(16))) float red[NW * BM * S::kRowF32];
 
   const int lane = threadIdx.x & 63;
@@ -66,6 +76,9 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs a) {
   const int s0 = wave * ksteps / NW, s1 = (wave + 1) * ksteps / NW;
   const rsrc_t xr = make_rsrc_uniform(a.x, 0x7ffffff0);
   const rsrc_t wr = make_rsrc_uniform(a.w, 0x7ffffff0);
+  // RoPE: the first output column of the workgroup's first half (BN / 2
+  // columns of a head's first 32).
+  auto rope_col = [](int n) { return n / 64 * 64 + n % 64 / 2; };
   // Byte offsets of this lane's rows at k-chunk q of k-step 0 (rows past M
   // or N read the last row: computed, never stored).
   unsigned xo[FM], wo[FN];
@@ -73,7 +86,9 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs a) {
   for (int j = 0; j < FM; ++j) xo[j] = (unsigned)((int64_t)min(m0 + j * 16 + r16, a.M - 1) * a.ldx * 2 + q * 16);
 #pragma unroll
   for (int i = 0; i < FN; ++i) {
-    const int n = min(n0 + i * 16 + r16, a.N - 1);
+    constexpr int kHalf = FN < 2 ? 1 : FN / 2;  // blocks of a half
+    const int col = kRope ? rope_col(n0) + i / kHalf * 32 + i % kHalf * 16 : n0 + i * 16;
+    const int n = min(col + r16, a.N - 1);
     wo[i] = a.w_kt ? (unsigned)((n / kBlkRows) * a.w_kt * kBlkBytes + (n % kBlkRows) * (kBlkK * 2) + q * 16)
                    : (unsigned)((int64_t)n * a.ldw * 2 + q * 16);
   }
@@ -88,16 +103,17 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs a) {
     for (int j = 0; j < FM; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 
   // Output vectors (8 columns of one row) per thread in the epilogue below.
-  constexpr int kOutCols = kGated ? BN / 2 : BN;
+  // (RoPE: 8 columns of the first half and the 8 that they rotate with)
+  constexpr int kOutCols = kGated || kRope ? BN / 2 : BN;
   constexpr int kVecs = kOutCols / 8;
-  const int out_n0 = kGated ? n0 / 2 : n0;
+  const int out_n0 = kRope ? rope_col(n0) : kGated ? n0 / 2 : n0;
   // When every thread has at most one output vector, its residual is
   // loaded now, before the k-loop: it depends on nothing the kernel
   // computes, and the epilogue then does not wait a memory round trip for
   // it.  (The thread reads exactly the elements it later writes, so y may
   // alias the residual.)
   // The bias (bias epilogues) likewise.
-  constexpr bool kOnePerThread = !kGated && BM * kVecs <= NW * 64;
+  constexpr bool kOnePerThread = !kGated && !kRope && BM * kVecs <= NW * 64;
   constexpr bool kResPre = epi_has_resid<E>() && kOnePerThread;
   constexpr bool kBiasPre = epi_has_bias<E>() && kOnePerThread;
   bf16x8 res_pre = {}, bias_pre = {};
@@ -108,6 +124,23 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs a) {
       if constexpr (kResPre) res_pre = load8_bf16(a.resid + (int64_t)m * a.ldr + n, a.Nout - n);
       if constexpr (kBiasPre) bias_pre = load8_bf16(a.bias + n, a.Nout - n);
     }
+  }
+  // The rotary cosines and sines of the thread's token and columns, two
+  // dependent reads, likewise.
+  constexpr bool kRopePre = kRope && BM * kVecs <= NW * 64;
+  f32x4 cos_pre[2] = {}, sin_pre[2] = {};
+  auto rope_load = [&](int m, int c, f32x4* cs, f32x4* sn) {  // c: column within the half head
+    const int pos = min(max(a.pos[m], 0), a.rope_rows - 1);  // stay inside the tables
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      cs[h] = *reinterpret_cast<const f32x4*>(a.rope_cos + (int64_t)pos * 32 + c + 4 * h);
+      sn[h] = *reinterpret_cast<const f32x4*>(a.rope_sin + (int64_t)pos * 32 + c + 4 * h);
+    }
+  };
+  if constexpr (kRopePre) {
+    const int t = threadIdx.x;
+    if (t < BM * kVecs && m0 + t / kVecs < a.M)
+      rope_load(m0 + t / kVecs, out_n0 % 64 + (t % kVecs) * 8, cos_pre, sin_pre);
   }
   // LayerNorm's column sums likewise.
   constexpr bool kColPre = NORM == kNormLayer && kOnePerThread;
@@ -247,9 +280,10 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs a) {
         v[e] += p0[e];
         v[4 + e] += p1[e];
       }
-      if constexpr (kGated) {  // the up rows of the same columns, 16 rows further
-        const f32x4 u0 = *reinterpret_cast<const f32x4*>(row + pc + 16);
-        const f32x4 u1 = *reinterpret_cast<const f32x4*>(row + pc + 20);
+      if constexpr (kGated || kRope) {  // the up rows of the same columns, 16 rows further; the second half
+        constexpr int kPartner = kGated ? 16 : BN / 2;
+        const f32x4 u0 = *reinterpret_cast<const f32x4*>(row + pc + kPartner);
+        const f32x4 u1 = *reinterpret_cast<const f32x4*>(row + pc + kPartner + 4);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           g[e] += u0[e];
@@ -257,7 +291,35 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs a) {
         }
       }
     }
-    // (for gated epilogues v holds the gate sums and g the up sums)
+    // (for gated epilogues v holds the gate sums and g the up sums; for RoPE
+    // the first and second half of a head)
+    if constexpr (kRope) {
+      // The rotation of src/kernels/modernbert.cu:31-74 on the bf16-rounded
+      // projection, rounded once; q, k and v go to their planes.
+      const int H = a.Nout / 3, p = n / H;
+      bf16x8 lo, hi;
+      if (p < 2) {
+        f32x4 cs[2], sn[2];
+        if constexpr (kRopePre) {
+          cs[0] = cos_pre[0], cs[1] = cos_pre[1], sn[0] = sin_pre[0], sn[1] = sin_pre[1];
+        } else {
+          rope_load(m, n % 64, cs, sn);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float x0 = round_bf16(v[e]), x1 = round_bf16(g[e]), c = cs[e / 4][e % 4], s = sn[e / 4][e % 4];
+          lo[e] = to_bf16(x0 * c - x1 * s);
+          hi[e] = to_bf16(x0 * s + x1 * c);
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) lo[e] = to_bf16(v[e]), hi[e] = to_bf16(g[e]);
+      }
+      __bf16* dst = a.y + p * a.plane + (int64_t)m * a.ldy + (n - p * H);
+      store8(dst, lo, 8);
+      store8(dst + 32, hi, 8);
+      continue;
+    }
     if constexpr (NORM != kNormNone) {
       const float mu = red[r * S::kRowF32 + BN + 2], rs = red[r * S::kRowF32 + BN + 3];
 #pragma unroll

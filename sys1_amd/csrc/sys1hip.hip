@@ -394,6 +394,13 @@ int64_t halo_rows(const KernelEntry& e, int64_t M, int halo) {
 constexpr int64_t kSkinnyMaxM = 4096;
 constexpr int64_t kSkinnyWeightBytes = 32 << 20;
 constexpr int64_t kSkinnyCuBytes = 704 << 10;
+// With RoPE, whose tile and stream-K plans are the head-aligned ones: up to
+// 64x64 skinny tiles won (us, against those plans: hidden 768 at 1 / 61 /
+// 300 / 400 tokens 5.5 / 6.1 / 9.1 / 9.7 against 11.7 / 19.0 / 12.4 / 12.5;
+// hidden 1024 at 16 / 300 tokens 6.5 / 11.2 against 11.2 / 14.2), 128x64
+// ones tied or lost (768 at 600: 12.9 against 12.6, 1024 at 600: 16.8
+// against 14.7).
+constexpr int64_t kSkinnyRopeCuBytes = 256 << 10;
 
 // The skinny kernels address x and w through one buffer descriptor each,
 // based at row 0, with 32-bit byte offsets: a call whose operands span 2 GiB
@@ -413,14 +420,16 @@ int skinny_pick(const Context* c, int64_t M, int64_t N, int64_t K, bool wide, in
     const int64_t bytes = (e.bm + e.bn) * K * 2;
     if (best < 0 || bytes < best_bytes) best = id, best_bytes = bytes;
   }
-  return best >= 0 && best_bytes <= kSkinnyCuBytes ? best : -1;
+  return best >= 0 && best_bytes <= (epi == kEpiRopeQkv ? kSkinnyRopeCuBytes : kSkinnyCuBytes) ? best : -1;
 }
 
 Plan price_plans(const Context* c, int64_t M0, int64_t N, int64_t K, bool wide, int epi, bool head64,
                  bool conv) {
   Plan best;
-  // (a forced grid or split asks for a persistent kernel: no skinny pick)
-  if (c->forced_kernel < 0 && c->forced_grid <= 0 && c->forced_dp < 0 && !head64 && !conv) {
+  // (a forced grid or split asks for a persistent kernel: no skinny pick;
+  // head64, the RoPE epilogue, is built for the skinny shapes of half or
+  // whole heads)
+  if (c->forced_kernel < 0 && c->forced_grid <= 0 && c->forced_dp < 0 && !conv) {
     const int id = skinny_pick(c, M0, N, K, wide, epi);
     if (id >= 0) {
       best.kernel = id, best.grid = cdiv(M0, kKernels[id].bm) * cdiv(N, kKernels[id].bn), best.dp = 0,

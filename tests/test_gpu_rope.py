@@ -153,3 +153,25 @@ def test_rope_qkv_errors(dev):
     with pytest.raises(ValueError):
         rq(x, torch.zeros(4, dtype=torch.int64, device="cuda"))
     assert rq(x, torch.zeros(4, dtype=torch.int32, device="cuda")).shape == (3, 4, 128)
+
+
+@pytest.mark.parametrize("hidden,heads", [(768, 12), (1024, 16), (200, 1), (256, 5)])
+def test_rope_qkv_of_small_batches(dev, orc, hidden, heads):
+    """The skinny kernels' RoPE (half and whole heads per workgroup), over the
+    token counts whose plans are their shapes, ragged last tile rows and K
+    not a multiple of a k-step.  The elementwise bound of the file's head."""
+    from sys1_amd.batching import draw_lengths, positions
+    from sys1_amd.rope import RopeQkvLinear
+    cos, sin = orc.rope_tables(160000.0, 64, 512)
+    w = orc.fill_normal((3 * heads * 64, hidden), 12, 0.02)
+    rq = RopeQkvLinear(to_gpu_bf16(w, torch), heads, torch.from_numpy(cos).cuda(), torch.from_numpy(sin).cuda(),
+                       device=dev)
+    for M in (1, 16, 17, 61, 129, 200, 260, 385, 512, 701):
+        lengths = draw_lengths(M, 1, min(M, 300), M, exact=True)
+        pos = positions(lengths)
+        x = orc.fill_normal((M, hidden), 20 + M)
+        print(f"[gpu] rope small hidden={hidden} heads={heads} M={M}", flush=True)
+        exp, proj = _expected(orc, x, w, cos, sin, pos, heads)
+        got = to_np(rq(to_gpu_bf16(x, torch), torch.from_numpy(pos).cuda()))
+        for p in range(3):
+            _check(orc, got[p], exp[p], f"M={M} plane {p}", _pair_norm(proj, p, heads) if p < 2 else None)
