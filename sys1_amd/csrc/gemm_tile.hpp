@@ -230,9 +230,14 @@ struct TileWalk {
 // for their partial stores (before the arrival counter) without draining
 // the refills in flight: a wave's vmcnt covers every vector memory access
 // it issued, and with producer waves those are its stores alone.
-template <int BM, int BN, int WM, int WN, int STAGES, int BK_, int OCC, bool STREAMK, int EPI, int PW = 0>
-__global__ __launch_bounds__((WM * WN + PW) * 64)
-__attribute__((amdgpu_waves_per_eu(((WM * WN + PW) * OCC + 3) / 4))) void gemm_tile_kernel(GemmArgs a) {
+// PW < 0: the ping-pong schedule (see below), STAGES its ring's slots.
+constexpr int producer_waves(int pw) { return pw > 0 ? pw : 0; }
+template <int BM, int BN, int WM, int WN, int STAGES_, int BK_, int OCC, bool STREAMK, int EPI, int PW_ = 0>
+__global__ __launch_bounds__((WM * WN + producer_waves(PW_)) * 64)
+__attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) / 4))) void gemm_tile_kernel(GemmArgs a) {
+  constexpr bool kPP = PW_ < 0;
+  constexpr int PW = producer_waves(PW_);
+  constexpr int STAGES = kPP ? 2 : STAGES_;
   using S = TileShape<BM, BN, WM, WN, STAGES, BK_>;
   constexpr int BK = S::BK;
   // Residual epilogues of producer-wave tile kernels whose LDS budget has
@@ -250,7 +255,10 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + PW) * OCC + 3) / 4))) void gemm_t
   // 378.5); in the compute waves they spilled (58.0 and 459.4 us).
   constexpr bool kStatPass = !STREAMK || epi_base(EPI) == kEpiConvSilu;
   constexpr int kOwnNorm = kStatPass ? kNormNone : epi_norm(EPI);
-  __shared__ __attribute__((aligned(1024))) char lds[S::kLdsBytes + kResBytes];
+  // (the ping-pong ring: STAGES_ slots of half the x or half the w rows)
+  constexpr int kSlotBytes = (BM > BN ? BM : BN) / 2 * S::kRowBytes;
+  static_assert(!kPP || STAGES_ * kSlotBytes <= 160 * 1024, "LDS budget of one gfx950 CU");
+  __shared__ __attribute__((aligned(1024))) char lds[kPP ? STAGES_ * kSlotBytes : S::kLdsBytes + kResBytes];
   char* const res_lds = lds + S::kLdsBytes;
   // (every k-tile loop needs two k-steps per tile, so that a tile's copy,
   // issued after its first barrier, lands before its last)
@@ -773,10 +781,13 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + PW) * OCC + 3) / 4))) void gemm_t
     // The bias of every column this lane stores, likewise loaded before
     // any store (the bias does not depend on the row: FN x 2 vectors).
     // (Only where the accumulators and the batched vectors take at most half
-    // of a wave's registers: beyond that the batch spills.)
+    // of a wave's registers: beyond that the batch spills.  The ping-pong
+    // kernel's fragment sets are free by then: with the bias of each row
+    // block read behind the last one's stores, the vision tower's fc1 at 8192
+    // rows ran 132 us, batched 119.)
     constexpr bool kBiasRegs = epi_has_bias<E>() && !epi_gated(E) && E != kEpiRopeQkv &&
-                               S::FM * S::FN * 16 + S::FN * 8 + (kResRegs ? S::FM * S::FN * 8 : 0) <=
-                                   512 / kWavesPerSimd / 2;
+                               (kPP || S::FM * S::FN * 16 + S::FN * 8 + (kResRegs ? S::FM * S::FN * 8 : 0) <=
+                                           512 / kWavesPerSimd / 2);
     bf16x8 rbias[kBiasRegs ? S::FN : 1][2];
     if constexpr (kBiasRegs) {
 #pragma unroll
@@ -1014,6 +1025,234 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + PW) * OCC + 3) / 4))) void gemm_t
     if (lane == 0) __hip_atomic_store(counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return true;
   };
+
+  // ---- ping-pong main loop (PW < 0), for large tiles and long streams.
+  //
+  // Two groups of four waves (one per SIMD each) run half a phase apart: in
+  // one barrier interval a wave reads the fragments of its next quadrant and
+  // issues its share of a refill, in the next it runs the quadrant's MFMAs
+  // (8 of 32 cycles at 256x256) while the SIMD's other wave loads.  A load
+  // that stalls its wave's issue then never stands in front of that wave's
+  // MFMAs, without producer waves and the third of the registers they hold.
+  //
+  // LDS is a ring of SLOTS slots of 16 KB.  A phase reads one unit (half of
+  // one operand's rows of a k-tile) and requests the unit kAhead phases on
+  // into the slot that the last phase freed: each operand byte is read from
+  // LDS once per wave, its slot is free a quarter of a k-tile later, and 2 1/4
+  // k-tiles are on their way at any time, against one in the two-stage
+  // 256x256 kernel that this replaces (its barrier waited for loads issued
+  // one k-tile before).
+  //
+  // Hazards.  A unit's readers wait for their reads (lgkmcnt(0)) before the
+  // barrier that ends their load interval; the first request into its slot
+  // is issued after the later group's.  A unit's requests have landed before
+  // it is read: each wave waits for its own share (vmcnt) one phase earlier,
+  // in front of a barrier that both groups pass before the first read.
+  //
+  // Measured, 8192 x 8192 x 8192: 1200 -> 1340-1397 TFLOP/s against the
+  // two-stage kernel, same boxes; 2010 with operands of zeros, so the rest is
+  // what the card's power allows for the data.
+  // Without its refills the loop reaches 2150, without its LDS reads 1730.
+  // Slower: the refills issued between the MFMAs (1163), before the fragment
+  // reads (1258), or half of each unit later (1220-1306); eight slots instead
+  // of ten lose up to 1%; the raster group (2 to 8 tile rows) changes nothing.
+  if constexpr (kPP) {
+    static_assert(WM == 2 && WN == 4 && BK == 64 && OCC == 1 && !STREAMK && !kConv, "ping-pong: 2 x 4 waves");
+    static_assert(S::FM % 2 == 0 && S::FN % 2 == 0, "ping-pong: wave tiles in quadrants");
+    constexpr int SLOTS = STAGES_;
+    constexpr int HM = S::FM / 2, HN = S::FN / 2;            // blocks of half a wave tile
+    constexpr int kXI = BM / 2 / S::RPI / S::kWaves;         // refill instructions per wave: half of x
+    constexpr int kWI = BN / 2 / S::RPI / S::kWaves;         // half of w
+    static_assert(kXI == kWI, "every unit is the same number of refill instructions");
+    static_assert(kXI * S::RPI * S::kWaves * 2 == BM && kWI * S::RPI * S::kWaves * 2 == BN, "refills deal evenly");
+    constexpr int kAhead = SLOTS - 1;                        // units requested ahead of the one read
+    // Unit u of the stream is half of one operand's rows of a k-tile, in the
+    // order x0, w0, w1, x1; the half h of x holds every wave row's blocks
+    // [h HM, (h + 1) HM), of w every wave column's [h HN, (h + 1) HN).
+    auto unit_row = [&](bool is_w, int h, int r) {  // unit row -> tile row
+      constexpr int hx = S::TM / 2, hw = S::TN / 2;
+      return is_w ? r / hw * S::TN + h * hw + r % hw : r / hx * S::TM + h * hx + r % hx;
+    };
+    unsigned soff[2 * (kXI + kWI)];
+    auto pp_offsets = [&](const Segment& sg) {
+      const int x_left = a.M - 1 - walk.row0(sg.tm), w_left = a.N - 1 - sg.tn * BN;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int i = 0; i < kXI; ++i) {
+          const int r = (i * S::kWaves + wave) * S::RPI + lrow;
+          soff[h * kXI + i] = (unsigned)(min(unit_row(false, h, r), x_left) * (int)a.ldx * 2 + ((lpos ^ lds_swz<BK>(r)) << 4));
+        }
+#pragma unroll
+        for (int i = 0; i < kWI; ++i) {
+          const int r = (i * S::kWaves + wave) * S::RPI + lrow, c = (lpos ^ lds_swz<BK>(r)) << 4;
+          const int rw = min(unit_row(true, h, r), w_left);
+          soff[2 * kXI + h * kWI + i] =
+              a.w_kt ? (unsigned)((rw / kBlkRows) * a.w_kt * kBlkBytes + (rw % kBlkRows) * (kBlkK * 2) + c)
+                     : (unsigned)(rw * (int)a.ldw * 2 + c);
+        }
+      }
+    };
+    const int steps = walk.steps();
+    // The request cursor: the descriptors of its k-tile, moved on by a
+    // scalar add per k-tile (in the shadow of a quadrant's MFMAs, not in
+    // front of a request).  Past the end of the stream a size of zero keeps
+    // the instruction count.
+    Segment qsg = walk.first_segment();
+    int qkt = qsg.kt0, qstep = 0;
+    const char *qx, *qw;
+    const int wstep = a.w_kt ? kBlkBytes : BK * 2;
+    auto enter_segment = [&]() {
+      const int n0 = qsg.tn * BN;
+      pp_offsets(qsg);
+      qx = reinterpret_cast<const char*>(a.x + (int64_t)walk.row0(qsg.tm) * a.ldx) + qsg.kt0 * BK * 2;
+      qw = a.w_kt ? reinterpret_cast<const char*>(a.w) + (int64_t)(n0 / kBlkRows) * a.w_kt * kBlkBytes
+                  : reinterpret_cast<const char*>(a.w + (int64_t)n0 * a.ldw);
+      qw += (int64_t)qsg.kt0 * wstep;
+    };
+    enter_segment();
+    int qbytes = 0x7ffffff0;
+    const int ktail = a.K % BK;  // valid k of a partial last k-tile
+    bool qtail = ktail && qsg.kt0 == walk.kt_count - 1;
+    // Request the cursor's unit of type T into `slot`.
+    auto request = [&](auto tc, int slot) {
+      constexpr int T = decltype(tc)::value;
+      constexpr bool is_w = T == 1 || T == 2;
+      constexpr int h = T >= 2 ? 1 : 0;
+      const rsrc_t r = make_rsrc_uniform(is_w ? qw : qx, qbytes);
+      unsigned off[kXI];
+#pragma unroll
+      for (int i = 0; i < kXI; ++i) off[i] = soff[is_w ? 2 * kXI + h * kWI + i : h * kXI + i];
+      if (qtail) {  // (wave-uniform) chunks past K read zeros
+#pragma unroll
+        for (int i = 0; i < kXI; ++i)
+          if ((lpos ^ lds_swz<BK>((i * S::kWaves + wave) * S::RPI + lrow)) * 8 >= ktail) off[i] = kOutOfRange;
+      }
+#pragma unroll
+      for (int i = 0; i < kXI; ++i)
+        dma16(r, off[i], (lds_void*)(lds + slot * kSlotBytes + (i * S::kWaves + wave) * 1024));
+    };
+    auto advance = [&](auto tc) {  // behind the request of type T
+      if constexpr (decltype(tc)::value == 3) {
+        qx += BK * 2;
+        qw += wstep;
+        if (++qstep >= steps) {
+          qbytes = 0;
+        } else if (++qkt == qsg.kt1) {
+          qsg = walk.next_segment(qsg);
+          qkt = qsg.kt0;
+          enter_segment();
+        }
+        qtail = ktail && qkt == walk.kt_count - 1;
+      }
+    };
+    constexpr int kInFlight = kXI * (kAhead - 1);  // refill instructions that may be outstanding at a barrier
+    static_assert(kInFlight < 64, "vmcnt field");
+
+    // Fragments: chunk 2 ks + fk of unit row r at ((fk ^ swz) << 4) ^ (ks << 5).
+    i32x4 xf[2][HM][S::KS], wf[2][HN][S::KS];
+    const int xr0 = wm * (S::TM / 2) + frow, wr0 = wn * (S::TN / 2) + frow;
+    const int xb = xr0 * S::kRowBytes + ((fk ^ lds_swz<BK>(xr0)) << 4);
+    const int wb = wr0 * S::kRowBytes + ((fk ^ lds_swz<BK>(wr0)) << 4);
+    // (32 rows further on, lds_swz flips its bit 2: the chunk of k-step ks ^ 2)
+    auto read_x = [&](int h, int slot) {
+      const int b = xb + slot * kSlotBytes;
+#pragma unroll
+      for (int j = 0; j < HM; ++j)
+#pragma unroll
+        for (int ks = 0; ks < S::KS; ++ks)
+          xf[h][j][ks] = *reinterpret_cast<const i32x4*>(lds + (b ^ ((ks ^ (j % 2 * 2)) << 5)) + j * 32 * S::kRowBytes);
+    };
+    auto read_w = [&](int h, int slot) {
+      const int b = wb + slot * kSlotBytes;
+#pragma unroll
+      for (int i = 0; i < HN; ++i)
+#pragma unroll
+        for (int ks = 0; ks < S::KS; ++ks)
+          wf[h][i][ks] = *reinterpret_cast<const i32x4*>(lds + (b ^ ((ks ^ (i % 2 * 2)) << 5)) + i * 32 * S::kRowBytes);
+    };
+    auto quadrant = [&](int hx, int hw) {
+#pragma unroll
+      for (int ks = 0; ks < S::KS; ++ks)
+#pragma unroll
+        for (int i = 0; i < HN; ++i)
+#pragma unroll
+          for (int j = 0; j < HM; ++j)
+            acc[hw * HN + i][hx * HM + j] = mfma32(wf[hw][i][ks], xf[hx][j][ks], acc[hw * HN + i][hx * HM + j]);
+    };
+    auto bar = [&]() {
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    int slot = 0, freed = SLOTS - 1;
+    auto next_slot = [&]() {
+      freed = slot;
+      slot = slot + 1 == SLOTS ? 0 : slot + 1;
+    };
+    // One phase of unit type T: its fragments, a request into the slot the
+    // last phase freed, the wait for the next phase's unit; the barrier; the
+    // quadrant that the fragments complete; the barrier.
+    auto phase = [&](auto tc, bool load, bool mul) {
+      constexpr int T = decltype(tc)::value;
+      if (load) {
+        if constexpr (T == 0) read_x(0, slot);
+        if constexpr (T == 1) read_w(0, slot);
+        if constexpr (T == 2) read_w(1, slot);
+        if constexpr (T == 3) read_x(1, slot);
+        __builtin_amdgcn_sched_barrier(0);
+        request(std::integral_constant<int, (T + kAhead) % 4>(), freed);
+        __builtin_amdgcn_sched_barrier(0);
+        next_slot();
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the slot just read may be refilled after the barrier
+        vm_wait<kInFlight>();
+      }
+      bar();
+      __builtin_amdgcn_s_setprio(1);
+      if (mul) {
+        if constexpr (T == 0) quadrant(1, 0);
+        if constexpr (T == 1) quadrant(0, 0);
+        if constexpr (T == 2) quadrant(0, 1);
+        if constexpr (T == 3) quadrant(1, 1);
+      }
+      if (load) advance(std::integral_constant<int, (T + kAhead) % 4>());
+      __builtin_amdgcn_s_setprio(0);
+      bar();
+    };
+    using std::integral_constant;
+    // Prologue: the first kAhead units, the first of them landed.
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      if (u % 4 == 0) request(integral_constant<int, 0>(), u);
+      if (u % 4 == 1) request(integral_constant<int, 1>(), u);
+      if (u % 4 == 2) request(integral_constant<int, 2>(), u);
+      if (u % 4 == 3) request(integral_constant<int, 3>(), u);
+      if (u % 4 == 3) advance(integral_constant<int, 3>());
+    }
+    vm_wait<kInFlight>();
+    bar();
+    const bool second = wave >= S::kWaves / 2;  // the group half a phase behind
+    if (second) bar();
+    Segment csg = walk.first_segment();
+    int ckt = csg.kt0;
+    for (int s = 0; s < steps; ++s) {
+      phase(integral_constant<int, 0>(), true, s > 0);
+      if (s > 0 && ++ckt == csg.kt1) {
+        epilogue(walk.row0(csg.tm), csg.tn * BN, 0);
+        zero_acc();
+        csg = walk.next_segment(csg);
+        ckt = csg.kt0;
+      }
+      phase(integral_constant<int, 1>(), true, true);
+      phase(integral_constant<int, 2>(), true, true);
+      phase(integral_constant<int, 3>(), true, true);
+    }
+    phase(integral_constant<int, 0>(), false, true);
+    epilogue(walk.row0(csg.tm), csg.tn * BN, 0);
+    if (!second) bar();
+    vm_wait<0>();  // the zero-size refills of the last units write LDS too
+    return;
+  }
 
   // ---- main loop over this workgroup's k-tile stream.  Step s lives in
   // stage s % STAGES.  The prologue requests steps 0..STAGES-1; after the

@@ -143,7 +143,7 @@ namespace {
 // Output-tile shapes, in the order of shapes.def (the kernel ids).
 const KernelEntry kKernels[] = {
 #define SYS1_SHAPE(name, BM, BN, WM, WN, ST, BK, OCC, SK, PW, EFF, SWEFF, LKEFF) \
-  KernelEntry{#name, BM, BN, (WM * WN + PW) * 64, OCC, SK, EFF, BK, ST, BN / WN, WM, PW, SWEFF, LKEFF, sys1::name##_fns, false},
+  KernelEntry{#name, BM, BN, (WM * WN + (PW > 0 ? PW : 0)) * 64, OCC, SK, EFF, BK, ST, BN / WN, WM, PW, SWEFF, LKEFF, sys1::name##_fns, false},
 // (skinny entries: tn 16 and wm 0 keep the RoPE and fused-conv calls off them)
 #define SYS1_SKINNY(name, FM, FN, NW, U) \
   KernelEntry{#name, 16 * FM, 16 * FN, NW * 64, 1, false, 1.0f, 32, 0, 16, 0, 0, 0.0f, 0.0f, sys1::name##_fns, true},
@@ -423,6 +423,12 @@ int skinny_pick(const Context* c, int64_t M, int64_t N, int64_t K, bool wide, in
   return best >= 0 && best_bytes <= (epi == kEpiRopeQkv ? kSkinnyRopeCuBytes : kSkinnyCuBytes) ? best : -1;
 }
 
+// The ping-pong shape is offered above this many tokens: with fewer 256-row
+// panels the weight stream decides.  Forced on the decoder widths it lost
+// 12-65% everywhere at 320 and 512 tokens; at 768 it gained 6-16% on the 27B
+// widths (in_proj 137.7 -> 118.2 us).
+constexpr int64_t kPingPongMinM = 640;
+
 Plan price_plans(const Context* c, int64_t M0, int64_t N, int64_t K, bool wide, int epi, bool head64,
                  bool conv) {
   Plan best;
@@ -474,6 +480,7 @@ Plan price_plans(const Context* c, int64_t M0, int64_t N, int64_t K, bool wide, 
       // split tile to fix up (measured: Qwen3.5-27B gate_up at M = 128,
       // 182 tiles of 128x192, 76.0 us against 81.6-84.1 us on the stream-K
       // hybrid whose 16 split tiles are summed after the stream).
+      if (e.pw < 0 && M <= kPingPongMinM) continue;
       const int64_t whole = cdiv(M, e.bm) * cdiv(N, e.bn);
       if (!e.streamk && M <= 128 &&
           !(M > 64 && cdiv(M, e.bm) == 1 && whole <= (int64_t)c->cus && 3 * whole >= 2 * (int64_t)c->cus))

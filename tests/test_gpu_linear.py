@@ -573,3 +573,37 @@ def test_blocked_weight_layout_is_bitwise_row_major(dev, orc):
                         assert torch.equal(g_rm(xg), g_bl(xg)), f"{name} swiglu"
     finally:
         dev.set_kernel(-1)
+
+
+@pytest.mark.parametrize("M,N,K,grid", [
+    (1, 8, 8, 0), (256, 256, 64, 0), (257, 264, 72, 0), (511, 520, 128, 1), (700, 800, 200, 2),
+    (1030, 520, 1032, 3), (513, 1284, 640, 5),
+])
+@pytest.mark.parametrize("blocked", [False, True])
+def test_ping_pong_tiles_at_their_edges(dev, orc, M, N, K, grid, blocked):
+    """The ping-pong kernel's unit stream: one to many k-tiles and tiles per
+    workgroup (forced grids run the ring across tile borders), ragged rows,
+    columns and K, both weight layouts; each element within one bf16 ulp of
+    the rounded float64 product, and the residual epilogue in place."""
+    from sys1_amd import kernel_names
+    from sys1_amd.linear import Linear
+    print(f"[gpu] ping-pong M={M} N={N} K={K} grid={grid} blocked={blocked}", flush=True)
+    x, w = _inputs(orc, M, N, K, 300 + M)
+    xb, wb = orc.round_bf16(x), orc.round_bf16(w)
+    ref = orc.linear_f64(xb, wb)
+    try:
+        dev.set_kernel(kernel_names().index("tile_256x256_s10_w2x4_pp"))
+        dev.set_grid(grid)
+        lin = Linear(to_gpu_bf16(w, torch), device=dev, blocked=blocked)
+        xg = to_gpu_bf16(x, torch)
+        y = lin(xg)
+        _check_close_to_rounded(orc, to_np(y), ref, "plain")
+        assert torch.equal(lin(xg), y)
+        h = to_gpu_bf16(orc.fill_normal((M, N), 9), torch)
+        p16 = orc.round_bf16(ref.astype(np.float32))
+        expect = orc.round_bf16(p16 + to_np(h))
+        lin.forward_into(xg, h, residual=h)
+        assert_parity(to_np(h), expect, "residual in place")
+    finally:
+        dev.set_kernel(-1)
+        dev.set_grid(0)
