@@ -11,8 +11,6 @@ With `norm_weight` the layer's input RMSNorm (:933) is fused as well.
 """
 from __future__ import annotations
 
-import ctypes
-
 import torch
 
 from . import _lib
@@ -20,7 +18,6 @@ from .device import HipDevice, load as load_device
 from .linear import _check_operand, _rows
 from .norm import fold_norm_weight
 
-_vp = ctypes.c_void_p
 
 
 class InProjConv:
@@ -50,28 +47,39 @@ class InProjConv:
         self.out_features, self.in_features = weight.shape
 
     def forward_into(self, x: torch.Tensor, positions: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
+        x2 = self._input(x, positions)
+        o2, _ = _rows(out, "out")
+        if o2.shape != (x2.shape[0], self.out_features):
+            raise ValueError(f"out must be [{x2.shape[0]}, {self.out_features}]")
+        self._project(x2, positions, o2)
+        return out
+
+    def _input(self, x: torch.Tensor, positions: torch.Tensor) -> torch.Tensor:
         _check_operand(x, "x", self.device)
         if x.shape[-1] != self.in_features:
             raise ValueError(f"shape mismatch: x[..., {x.shape[-1]}] vs K={self.in_features}")
         x2, _ = _rows(x, "x")
-        o2, _ = _rows(out, "out")
-        M, K = x2.shape
-        if o2.shape != (M, self.out_features):
-            raise ValueError(f"out must be [{M}, {self.out_features}]")
-        if positions.shape != (M,) or positions.dtype != torch.int32 or positions.device != x.device:
+        if positions.shape != (x2.shape[0],) or positions.dtype is not torch.int32 or positions.device != x.device:
             raise ValueError("positions must be int32 [M] on the input's device")
+        return x2
+
+    def _project(self, x2: torch.Tensor, positions: torch.Tensor, o2: torch.Tensor) -> None:
+        M, K = x2.shape
         dev = self.device
         dev.follow_torch_stream()
-        _lib.check(dev._L.sys1hip_linear_conv_silu_bf16(
-            dev.ctx, _vp(x2.data_ptr()), x2.stride(0) if M > 1 else K,
-            _vp(self.weight.data_ptr()), self.weight.stride(0), self.norm, self.eps,
-            _vp(self.conv_weight.data_ptr()), self.conv_channels, _vp(positions.data_ptr()),
-            _vp(o2.data_ptr()), o2.stride(0) if M > 1 else o2.shape[1],
-            M, self.out_features, K), dev.ctx)
-        return out
+        rc = dev._L.sys1hip_linear_conv_silu_bf16(
+            dev.ctx, x2.data_ptr(), x2.stride(0) if M > 1 else K,
+            self.weight.data_ptr(), self.weight.stride(0), self.norm, self.eps,
+            self.conv_weight.data_ptr(), self.conv_channels, positions.data_ptr(),
+            o2.data_ptr(), o2.stride(0) if M > 1 else o2.shape[1],
+            M, self.out_features, K)
+        if rc:
+            _lib.check(rc, dev.ctx)
 
     def forward(self, x: torch.Tensor, positions: torch.Tensor) -> torch.Tensor:
-        out = torch.empty(*x.shape[:-1], self.out_features, dtype=torch.bfloat16, device=x.device)
-        return self.forward_into(x, positions, out)
+        x2 = self._input(x, positions)
+        o2 = x2.new_empty((x2.shape[0], self.out_features))
+        self._project(x2, positions, o2)
+        return o2 if x.dim() == 2 else o2.view(*x.shape[:-1], self.out_features)
 
     __call__ = forward

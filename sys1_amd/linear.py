@@ -31,11 +31,11 @@ _vp = ctypes.c_void_p
 
 
 def _check_operand(t: torch.Tensor, name: str, dev: HipDevice) -> None:
-    if t.dtype != torch.bfloat16:
+    if t.dtype is not torch.bfloat16:
         raise ValueError(f"{name}: expected bf16, got {t.dtype}")
-    if t.device != dev.torch_device:
+    if t.get_device() != dev.index:  # (-1 for a CPU tensor)
         raise ValueError(f"{name}: expected a tensor on {dev.torch_device}, got {t.device}")
-    if t.dim() >= 1 and t.shape[-1] > 1 and t.stride(-1) != 1:
+    if t.dim() >= 1 and t.stride(-1) != 1 and t.shape[-1] > 1:
         raise ValueError(f"{name}: last dimension must be contiguous")
 
 
@@ -59,15 +59,18 @@ def linear_bf16(dev: HipDevice, x: torch.Tensor, w: torch.Tensor, out: torch.Ten
     blocked = bool(epilogue & _lib.EPI_BLOCKED_W)
     N = n if blocked else w.shape[0]
     dev.follow_torch_stream()
-    _lib.check(dev._L.sys1hip_linear_bf16(
+    # (plain integers for the pointers: a c_void_p object each costs ~0.2 us)
+    rc = dev._L.sys1hip_linear_bf16(
         dev.ctx,
-        _vp(x.data_ptr()), x.stride(0) if M > 1 else K,
-        _vp(w.data_ptr()), K if blocked else w.stride(0),
-        _vp(bias.data_ptr()) if bias is not None else None,
-        _vp(residual.data_ptr()) if residual is not None else None,
+        x.data_ptr(), x.stride(0) if M > 1 else K,
+        w.data_ptr(), K if blocked else w.stride(0),
+        bias.data_ptr() if bias is not None else None,
+        residual.data_ptr() if residual is not None else None,
         (residual.stride(0) if M > 1 else residual.shape[1]) if residual is not None else 0,
-        _vp(out.data_ptr()), out.stride(0) if M > 1 else out.shape[1],
-        M, N, K, epilogue), dev.ctx)
+        out.data_ptr(), out.stride(0) if M > 1 else out.shape[1],
+        M, N, K, epilogue)
+    if rc:
+        _lib.check(rc, dev.ctx)
     return out
 
 
@@ -119,7 +122,7 @@ class Linear:
         e = _lib.EPI_BLOCKED_W if self.blocked else _lib.EPI_NONE
         if self.bias is not None:
             e |= _lib.EPI_BIAS
-        if gelu not in (False, True, "erf", "tanh"):
+        if gelu is not False and gelu not in (False, True, "erf", "tanh"):
             raise ValueError(f"gelu must be False, True, 'erf' or 'tanh', got {gelu!r}")
         if gelu:
             if self.bias is None:
@@ -131,14 +134,21 @@ class Linear:
 
     def forward_into(self, x: torch.Tensor, out: torch.Tensor,
                      residual: torch.Tensor | None = None, gelu: bool | str = False) -> torch.Tensor:
+        x2 = self._input(x)
+        o2, _ = _rows(out, "out")
+        if o2.shape != (x2.shape[0], self.out_features):
+            raise ValueError(f"out must be [{x2.shape[0]}, {self.out_features}], got {tuple(out.shape)}")
+        self._project(x2, o2, residual, gelu)
+        return out
+
+    def _input(self, x: torch.Tensor) -> torch.Tensor:
         _check_operand(x, "x", self.device)
         if x.shape[-1] != self.in_features:
             raise ValueError(f"shape mismatch: x[..., {x.shape[-1]}] vs weight "
                              f"[{self.out_features}, {self.in_features}]")
-        x2, _ = _rows(x, "x")
-        o2, _ = _rows(out, "out")
-        if o2.shape != (x2.shape[0], self.out_features):
-            raise ValueError(f"out must be [{x2.shape[0]}, {self.out_features}], got {tuple(out.shape)}")
+        return _rows(x, "x")[0]
+
+    def _project(self, x2: torch.Tensor, o2: torch.Tensor, residual, gelu) -> None:
         r2 = None
         if residual is not None:
             _check_operand(residual, "residual", self.device)
@@ -147,12 +157,14 @@ class Linear:
                 raise ValueError(f"residual must match the output shape {tuple(o2.shape)}")
         linear_bf16(self.device, x2, self.weight, o2, self._epilogue(residual, gelu),
                     self.bias, r2, n=self.out_features)
-        return out
 
     def forward(self, x: torch.Tensor, residual: torch.Tensor | None = None,
                 gelu: bool | str = False) -> torch.Tensor:
-        out = torch.empty(*x.shape[:-1], self.out_features, dtype=torch.bfloat16, device=x.device)
-        return self.forward_into(x, out, residual, gelu)
+        # (an output made here needs none of forward_into's checks of it)
+        x2 = self._input(x)
+        o2 = x2.new_empty((x2.shape[0], self.out_features))
+        self._project(x2, o2, residual, gelu)
+        return o2 if x.dim() == 2 else o2.view(*x.shape[:-1], self.out_features)
 
     __call__ = forward
 
@@ -201,19 +213,23 @@ class GatedLinear:
         self.out_features = weight.shape[0] // 2
 
     def forward_into(self, x: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
-        _check_operand(x, "x", self.device)
-        if x.shape[-1] != self.in_features:
-            raise ValueError(f"shape mismatch: x[..., {x.shape[-1]}] vs K={self.in_features}")
-        x2, _ = _rows(x, "x")
+        x2 = self._input(x)
         o2, _ = _rows(out, "out")
         if o2.shape != (x2.shape[0], self.out_features):
             raise ValueError(f"out must be [{x2.shape[0]}, {self.out_features}]")
         return linear_bf16(self.device, x2, self.weight, o2, self.epilogue, n=self.rows)
 
+    def _input(self, x: torch.Tensor) -> torch.Tensor:
+        _check_operand(x, "x", self.device)
+        if x.shape[-1] != self.in_features:
+            raise ValueError(f"shape mismatch: x[..., {x.shape[-1]}] vs K={self.in_features}")
+        return _rows(x, "x")[0]
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        out = torch.empty(*x.shape[:-1], self.out_features, dtype=torch.bfloat16, device=x.device)
-        self.forward_into(x, out)
-        return out
+        x2 = self._input(x)
+        o2 = x2.new_empty((x2.shape[0], self.out_features))
+        linear_bf16(self.device, x2, self.weight, o2, self.epilogue, n=self.rows)
+        return o2 if x.dim() == 2 else o2.view(*x.shape[:-1], self.out_features)
 
     __call__ = forward
 

@@ -78,27 +78,37 @@ class NormLinear:
         self.out_features = weight.shape[0] // 2 if gated else weight.shape[0]
 
     def forward_into(self, x: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
+        x2 = self._input(x)
+        o2, _ = _rows(out, "out")
+        if o2.shape != (x2.shape[0], self.out_features):
+            raise ValueError(f"out must be [{x2.shape[0]}, {self.out_features}]")
+        self._project(x2, o2)
+        return out
+
+    def _input(self, x: torch.Tensor) -> torch.Tensor:
         _check_operand(x, "x", self.device)
         if x.shape[-1] != self.in_features:
             raise ValueError(f"shape mismatch: x[..., {x.shape[-1]}] vs K={self.in_features}")
-        x2, _ = _rows(x, "x")
-        o2, _ = _rows(out, "out")
+        return _rows(x, "x")[0]
+
+    def _project(self, x2: torch.Tensor, o2: torch.Tensor) -> None:
         M, K = x2.shape
-        if o2.shape != (M, self.out_features):
-            raise ValueError(f"out must be [{M}, {self.out_features}]")
         dev = self.device
         dev.follow_torch_stream()
-        _lib.check(dev._L.sys1hip_norm_linear_bf16(
-            dev.ctx, _vp(x2.data_ptr()), x2.stride(0) if M > 1 else K,
-            _vp(self.weight.data_ptr()), K if self.blocked else self.weight.stride(0),
-            _vp(self.colsum.data_ptr()) if self.colsum is not None else None,
+        rc = dev._L.sys1hip_norm_linear_bf16(
+            dev.ctx, x2.data_ptr(), x2.stride(0) if M > 1 else K,
+            self.weight.data_ptr(), K if self.blocked else self.weight.stride(0),
+            self.colsum.data_ptr() if self.colsum is not None else None,
             KINDS[self.kind], self.eps,
-            _vp(o2.data_ptr()), o2.stride(0) if M > 1 else o2.shape[1],
-            M, self.rows, K, self.epilogue | (_lib.EPI_BLOCKED_W if self.blocked else 0)), dev.ctx)
-        return out
+            o2.data_ptr(), o2.stride(0) if M > 1 else o2.shape[1],
+            M, self.rows, K, self.epilogue | (_lib.EPI_BLOCKED_W if self.blocked else 0))
+        if rc:
+            _lib.check(rc, dev.ctx)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        out = torch.empty(*x.shape[:-1], self.out_features, dtype=torch.bfloat16, device=x.device)
-        return self.forward_into(x, out)
+        x2 = self._input(x)
+        o2 = x2.new_empty((x2.shape[0], self.out_features))
+        self._project(x2, o2)
+        return o2 if x.dim() == 2 else o2.view(*x.shape[:-1], self.out_features)
 
     __call__ = forward

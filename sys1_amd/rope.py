@@ -17,14 +17,11 @@ device with torch.
 """
 from __future__ import annotations
 
-import ctypes
-
 import torch
 
 from . import _lib
 from .device import HipDevice, load as load_device
 
-_vp = ctypes.c_void_p
 HEAD_DIM = 64
 
 
@@ -68,24 +65,32 @@ class RopeQkvLinear:
         self.hidden = weight.shape[1]
 
     def forward_into(self, x: torch.Tensor, positions: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
-        if x.dtype != torch.bfloat16 or x.dim() != 2 or x.shape[1] != self.hidden or x.stride(1) != 1:
-            raise ValueError(f"x must be bf16 [M, {self.hidden}] with unit column stride")
-        M = x.shape[0]
-        if positions.dtype != torch.int32 or positions.shape != (M,) or not positions.is_contiguous():
-            raise ValueError("positions must be a contiguous int32 [M] tensor")
-        H = self.heads * HEAD_DIM
+        self._check(x, positions)
+        M, H = x.shape[0], self.heads * HEAD_DIM
         if out.dtype != torch.bfloat16 or tuple(out.shape) != (3, M, H) or not out.is_contiguous():
             raise ValueError(f"out must be a contiguous bf16 [3, {M}, {H}] tensor")
-        self.device.follow_torch_stream()
-        rc = self.device._L.sys1hip_linear_rope_qkv_bf16(
-            self.device.ctx, _vp(x.data_ptr()), x.stride(0), _vp(self.weight.data_ptr()),
-            self.weight.stride(0), _vp(self.cos.data_ptr()), _vp(self.sin.data_ptr()),
-            self.cos.shape[0], _vp(positions.data_ptr()), _vp(out.data_ptr()), M, self.heads, HEAD_DIM, self.hidden)
-        _lib.check(rc, self.device.ctx)
+        return self._project(x, positions, out)
+
+    def _check(self, x: torch.Tensor, positions: torch.Tensor) -> None:
+        if x.dtype is not torch.bfloat16 or x.dim() != 2 or x.shape[1] != self.hidden or x.stride(1) != 1:
+            raise ValueError(f"x must be bf16 [M, {self.hidden}] with unit column stride")
+        M = x.shape[0]
+        if positions.dtype is not torch.int32 or positions.shape != (M,) or not positions.is_contiguous():
+            raise ValueError("positions must be a contiguous int32 [M] tensor")
+
+    def _project(self, x: torch.Tensor, positions: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
+        dev = self.device
+        dev.follow_torch_stream()
+        rc = dev._L.sys1hip_linear_rope_qkv_bf16(
+            dev.ctx, x.data_ptr(), x.stride(0), self.weight.data_ptr(), self.weight.stride(0),
+            self.cos.data_ptr(), self.sin.data_ptr(), self.cos.shape[0], positions.data_ptr(), out.data_ptr(),
+            x.shape[0], self.heads, HEAD_DIM, self.hidden)
+        if rc:
+            _lib.check(rc, dev.ctx)
         return out
 
     def forward(self, x: torch.Tensor, positions: torch.Tensor) -> torch.Tensor:
-        out = torch.empty(3, x.shape[0], self.heads * HEAD_DIM, dtype=torch.bfloat16, device=x.device)
-        return self.forward_into(x, positions, out)
+        self._check(x, positions)
+        return self._project(x, positions, x.new_empty((3, x.shape[0], self.heads * HEAD_DIM)))
 
     __call__ = forward
