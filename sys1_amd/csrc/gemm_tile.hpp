@@ -751,6 +751,41 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) /
     }
     const int h = fk;
     const int out_n0 = epi_gated(E) ? (n0 + wn * S::TN) / 2 : n0 + wn * S::TN;
+    // Outputs, residuals and biases of calls whose rows are all 16-byte
+    // aligned and within 2 GiB move by buffer instructions: a 32-bit row
+    // offset per row block, the column in the instruction, rows past M
+    // dropped by the descriptor's size.  The others take the element-wise
+    // checks of store8 and load8, which cost a 64-bit address, an alignment
+    // test and a divergent branch per 16 bytes (the vision tower's fc1 at 3001
+    // rows 43.7 -> 39.8 us, 27B gate_up at 4096 tokens 1162 -> 1128, where the
+    // ping-pong groups' epilogues follow each other; 256x160 plans 0-2%).
+    const bool vec_n = a.Nout % 8 == 0;
+    const bool vec_y = vec_n && a.ldy % 8 == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0 &&
+                       ((int64_t)a.M + BM) * a.ldy * 2 < 0x7ffffff0ll;  // (no row of a tile wraps 32 bits)
+    const bool vec_r = epi_has_resid<E>() && vec_n && a.ldr % 8 == 0 &&
+                       (reinterpret_cast<uintptr_t>(a.resid) & 15) == 0 &&
+                       ((int64_t)a.M + BM) * a.ldr * 2 < 0x7ffffff0ll;
+    const bool vec_b = epi_has_bias<E>() && vec_n && (reinterpret_cast<uintptr_t>(a.bias) & 15) == 0;
+    const rsrc_t yr = make_rsrc(a.y, vec_y ? (int)((int64_t)a.M * a.ldy * 2) : 0);
+    const rsrc_t rr = make_rsrc(a.resid, vec_r ? (int)((int64_t)a.M * a.ldr * 2) : 0);
+    const rsrc_t br = make_rsrc(a.bias, vec_b ? a.Nout * 2 : 0);
+    auto put = [&](int m, int n, bf16x8 v) {
+      if (vec_y)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, v), yr,
+                                               n < a.Nout ? (int)(m * (int)a.ldy * 2 + n * 2) : (int)kOutOfRange, 0, 0);
+      else if (m < a.M && n < a.Nout)
+        store8(a.y + (int64_t)m * a.ldy + n, v, a.Nout - n);
+    };
+    auto get_resid = [&](int m, int n) -> bf16x8 {
+      if (vec_r)
+        return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(
+            rr, n < a.Nout ? (int)(m * (int)a.ldr * 2 + n * 2) : (int)kOutOfRange, 0, 0));
+      return m < a.M && n < a.Nout ? load8_bf16(a.resid + (int64_t)m * a.ldr + n, a.Nout - n) : bf16x8{};
+    };
+    auto get_bias = [&](int n) -> bf16x8 {
+      if (vec_b) return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(br, n * 2, 0, 0));
+      return n < a.Nout ? load8_bf16(a.bias + n, a.Nout - n) : bf16x8{};
+    };
     // The residual of every element this lane stores, loaded before any
     // store: y may alias it (the in-place update of the hidden state), and a
     // load behind a store to a possibly aliasing address would wait a whole
@@ -772,8 +807,7 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) /
 #pragma unroll
             for (int gp = 0; gp < 2; ++gp) {
               const int n = out_n0 + i * 32 + 16 * gp + 8 * h;
-              rres[j][i][gp] = m < a.M && n < a.Nout ? load8_bf16(a.resid + (int64_t)m * a.ldr + n, a.Nout - n)
-                                                     : bf16x8{};
+              rres[j][i][gp] = get_resid(m, n);
             }
         }
       }
@@ -795,7 +829,7 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) /
 #pragma unroll
         for (int gp = 0; gp < 2; ++gp) {
           const int n = out_n0 + i * 32 + 16 * gp + 8 * h;
-          rbias[i][gp] = n < a.Nout ? load8_bf16(a.bias + n, a.Nout - n) : bf16x8{};
+          rbias[i][gp] = get_bias(n);
         }
     }
 #pragma unroll
@@ -866,8 +900,7 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) /
             for (int e = 0; e < 4; ++e)
               o[g][e] = to_bf16(epi_gate<E>(acc[i][j][4 * g + e], acc[i][j][4 * (g + 2) + e]));
           const bf16x8 v = pair16(o[0], o[1]);
-          const int n = out_n0 + i * 16 + 8 * h;
-          if (row_ok && n < a.Nout) store8(a.y + (int64_t)m * a.ldy + n, v, a.Nout - n);
+          put(m, out_n0 + i * 16 + 8 * h, v);
         } else {
 #pragma unroll
           for (int gp = 0; gp < 2; ++gp) {
@@ -878,39 +911,23 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) /
               for (int e = 0; e < 4; ++e) p[q][e] = to_bf16(acc[i][j][4 * (2 * gp + q) + e]);
             bf16x8 v = pair16(p[0], p[1]);
             const int n = out_n0 + i * 32 + 16 * gp + 8 * h;
-            if (row_ok && n < a.Nout) {
-              const int valid = a.Nout - n;
-              if constexpr (E != kEpiNone) {
-                float b[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-                if constexpr (kBiasRegs) {
-#pragma unroll
-                  for (int e = 0; e < 8; ++e) b[e] = to_f32(rbias[i][gp][e]);
-                } else if constexpr (epi_has_bias<E>()) {
-                  load8(a.bias + n, b, valid);
-                }
-                float r[8];
-                if constexpr (epi_has_resid<E>()) {
-                  if (kResLds && res_in_lds) {
-                    const bf16x8 rv = *reinterpret_cast<const bf16x8*>(
-                        res_lds + ((m - m0) * BN + (n - n0)) * 2);
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) r[e] = to_f32(rv[e]);
-                  } else if constexpr (kResRegs) {
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) r[e] = to_f32(rres[j][i][gp][e]);
-                  } else {
-                    load8(a.resid + (int64_t)m * a.ldr + n, r, valid);
-                  }
-                }
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                  float t = epi_pre<E>(to_f32(v[e]), b[e]);
-                  if constexpr (epi_has_resid<E>()) t = round_bf16(t + r[e]);
-                  v[e] = to_bf16(t);
-                }
+            if constexpr (E != kEpiNone) {
+              bf16x8 b = {}, r = {};
+              if constexpr (kBiasRegs) b = rbias[i][gp];
+              else if constexpr (epi_has_bias<E>()) b = get_bias(n);
+              if constexpr (epi_has_resid<E>()) {
+                if (kResLds && res_in_lds) r = *reinterpret_cast<const bf16x8*>(res_lds + ((m - m0) * BN + (n - n0)) * 2);
+                else if constexpr (kResRegs) r = rres[j][i][gp];
+                else r = get_resid(m, n);
               }
-              store8(a.y + (int64_t)m * a.ldy + n, v, valid);
+#pragma unroll
+              for (int e = 0; e < 8; ++e) {
+                float t = epi_pre<E>(to_f32(v[e]), to_f32(b[e]));
+                if constexpr (epi_has_resid<E>()) t = round_bf16(t + to_f32(r[e]));
+                v[e] = to_bf16(t);
+              }
             }
+            put(m, n, v);
           }
         }
       }

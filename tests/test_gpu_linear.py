@@ -607,3 +607,41 @@ def test_ping_pong_tiles_at_their_edges(dev, orc, M, N, K, grid, blocked):
     finally:
         dev.set_kernel(-1)
         dev.set_grid(0)
+
+
+@pytest.mark.parametrize("name", ["tile_128x192_s3_w4x2_p4", "tile_256x256_s10_w2x4_pp", "stream_64x256_s4_w2x4_p4"])
+@pytest.mark.parametrize("M,N,ld,off", [
+    (3, 200, 200, 0),            # every row 16-byte aligned
+    (130, 200, 208, 8),          # a column slice, aligned
+    (130, 200, 204, 0),          # rows not 16-byte aligned
+    (130, 200, 208, 4),          # base not 16-byte aligned
+    (130, 197, 208, 0),          # ragged columns
+    (2, 200, 1 << 29, 0),        # row offsets past 32 bits: a tile row 4 would wrap onto row 0
+])
+def test_epilogue_addressing(dev, orc, name, M, N, ld, off):
+    """The epilogue's buffer-addressed outputs and residuals and the checked
+    element-wise ones: in place over a strided view, nothing outside it
+    touched, each output within one bf16 ulp of the rounded sum."""
+    from sys1_amd import kernel_names
+    from sys1_amd.linear import Linear
+    K = 128
+    print(f"[gpu] epilogue addressing {name} M={M} N={N} ld={ld} off={off}", flush=True)
+    x, w = _inputs(orc, M, N, K, 900 + M)
+    p16 = orc.round_bf16(orc.linear_f64(orc.round_bf16(x), orc.round_bf16(w)).astype(np.float32))
+    res = orc.round_bf16(orc.fill_normal((M, N), 17))
+    buf = torch.full(((M - 1) * ld + off + N + 64,), 7.0, dtype=torch.bfloat16, device="cuda:0")
+    h = buf[off:].as_strided((M, N), (ld, 1))
+    h.copy_(to_gpu_bf16(res, torch))
+    try:
+        dev.set_kernel(kernel_names().index(name))
+        Linear(to_gpu_bf16(w, torch), device=dev).forward_into(to_gpu_bf16(x, torch), h, residual=h)
+        ref = orc.round_bf16(p16 + res)
+        y = to_np(h)
+        assert (np.abs(y - ref) <= bf16_ulp(ref) + bf16_ulp(p16) + 1e-6).all()
+        assert (buf[:off] == 7.0).all()
+        if ld < 1 << 20:
+            gap = buf[off:off + (M - 1) * ld].reshape(M - 1, ld)[:, N:]
+            assert (gap == 7.0).all()
+        assert (buf[off + (M - 1) * ld + N:] == 7.0).all()
+    finally:
+        dev.set_kernel(-1)
