@@ -759,7 +759,11 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) /
     // test and a divergent branch per 16 bytes (the vision tower's fc1 at 3001
     // rows 43.7 -> 39.8 us, 27B gate_up at 4096 tokens 1162 -> 1128, where the
     // ping-pong groups' epilogues follow each other; 256x160 plans 0-2%).
-    const bool vec_n = a.Nout % 8 == 0;
+    // (Not for bias and residual together at three waves per SIMD, whose
+    // descriptors spill into the k-loop: vision fc2 on 256x160 104 -> 112 us.
+    // Nor beside the residual's LDS copy: 15 registers spill, not 4.)
+    constexpr bool kVec = kWavesPerSimd <= 2 || !(E == kEpiBiasResidual || kResLds);
+    const bool vec_n = kVec && a.Nout % 8 == 0;
     const bool vec_y = vec_n && a.ldy % 8 == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0 &&
                        ((int64_t)a.M + BM) * a.ldy * 2 < 0x7ffffff0ll;  // (no row of a tile wraps 32 bits)
     const bool vec_r = epi_has_resid<E>() && vec_n && a.ldr % 8 == 0 &&
@@ -832,76 +836,115 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) /
           rbias[i][gp] = get_bias(n);
         }
     }
-#pragma unroll
-    for (int j = 0; j < S::FM; ++j) {
+    // A block (i, j); cbias and cres are its bias and residual vectors where
+    // they were read in a batch of the column blocks' rows (kPipe).
+    constexpr bool kPipe = kWavesPerSimd <= 2 && !epi_gated(E) && E != kEpiRopeQkv &&
+                           ((epi_has_bias<E>() && !kBiasRegs) || (epi_has_resid<E>() && !kResRegs));
+    auto block = [&](int j, int i, const bf16x8* cbias, const bf16x8* cres) {
       const int m = m0 + wm * S::TM + j * 32 + frow;
       const bool row_ok = m < a.M;
+      if constexpr (E == kEpiRopeQkv) {
+        // Blocks i (even) and i+1 are the two halves of one 64-wide head
+        // (the plan guarantees 64-wide, head-aligned wave columns), so a
+        // lane holds columns c and c+32 of the same token: the rotation
+        // of src/kernels/modernbert.cu:31-74 happens in registers on the
+        // bf16-rounded projection, rounded once, and q, k and v go to
+        // their planes.
+        if (i % 2 == 0) {
+          const int nw = out_n0 + i * 32;  // head start column in qkv
+          const int H = a.Nout / 3;
+          const int p = nw / H;
+          const int col = nw - p * H;
+          const int pos = row_ok ? min(max(a.pos[m], 0), a.rope_rows - 1) : 0;  // stay inside the tables
+          bf16x4 lo[4], hi[4];
 #pragma unroll
-      for (int i = 0; i < S::FN; ++i) {
-        if constexpr (E == kEpiRopeQkv) {
-          // Blocks i (even) and i+1 are the two halves of one 64-wide head
-          // (the plan guarantees 64-wide, head-aligned wave columns), so a
-          // lane holds columns c and c+32 of the same token: the rotation
-          // of src/kernels/modernbert.cu:31-74 happens in registers on the
-          // bf16-rounded projection, rounded once, and q, k and v go to
-          // their planes.
-          if (i % 2 == 0) {
-            const int nw = out_n0 + i * 32;  // head start column in qkv
-            const int H = a.Nout / 3;
-            const int p = nw / H;
-            const int col = nw - p * H;
-            const int pos = row_ok ? min(max(a.pos[m], 0), a.rope_rows - 1) : 0;  // stay inside the tables
-            bf16x4 lo[4], hi[4];
+          for (int g = 0; g < 4; ++g) {
+            float x0[4], x1[4];
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-              float x0[4], x1[4];
-#pragma unroll
-              for (int e = 0; e < 4; ++e) {
-                x0[e] = round_bf16(acc[i][j][4 * g + e]);
-                x1[e] = round_bf16(acc[i + 1][j][4 * g + e]);
-              }
-              if (p < 2) {
-                const int c = 8 * g + 4 * h;  // column within the half head
-                const f32x4 cs = *reinterpret_cast<const f32x4*>(a.rope_cos + (int64_t)pos * 32 + c);
-                const f32x4 sn = *reinterpret_cast<const f32x4*>(a.rope_sin + (int64_t)pos * 32 + c);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                  const float r0 = x0[e] * cs[e] - x1[e] * sn[e];
-                  const float r1 = x0[e] * sn[e] + x1[e] * cs[e];
-                  x0[e] = r0;
-                  x1[e] = r1;
-                }
-              }
+            for (int e = 0; e < 4; ++e) {
+              x0[e] = round_bf16(acc[i][j][4 * g + e]);
+              x1[e] = round_bf16(acc[i + 1][j][4 * g + e]);
+            }
+            if (p < 2) {
+              const int c = 8 * g + 4 * h;  // column within the half head
+              const f32x4 cs = *reinterpret_cast<const f32x4*>(a.rope_cos + (int64_t)pos * 32 + c);
+              const f32x4 sn = *reinterpret_cast<const f32x4*>(a.rope_sin + (int64_t)pos * 32 + c);
 #pragma unroll
               for (int e = 0; e < 4; ++e) {
-                lo[g][e] = to_bf16(x0[e]);
-                hi[g][e] = to_bf16(x1[e]);
+                const float r0 = x0[e] * cs[e] - x1[e] * sn[e];
+                const float r1 = x0[e] * sn[e] + x1[e] * cs[e];
+                x0[e] = r0;
+                x1[e] = r1;
               }
             }
-            __bf16* dst = a.y + p * a.plane + (int64_t)m * a.ldy + col;
 #pragma unroll
-            for (int gp = 0; gp < 2; ++gp) {
-              const bf16x8 vlo = pair16(lo[2 * gp], lo[2 * gp + 1]);
-              const bf16x8 vhi = pair16(hi[2 * gp], hi[2 * gp + 1]);
-              if (row_ok) {
-                store8(dst + 16 * gp + 8 * h, vlo, 8);
-                store8(dst + 32 + 16 * gp + 8 * h, vhi, 8);
-              }
+            for (int e = 0; e < 4; ++e) {
+              lo[g][e] = to_bf16(x0[e]);
+              hi[g][e] = to_bf16(x1[e]);
             }
           }
-        } else if constexpr (epi_gated(E)) {
-          // A 32-row block of the packed weight is 16 gate rows then the 16
-          // up rows of the same 16 output columns: registers 4g+e (g = 0, 1)
-          // hold gate rows, 4(g+2)+e the matching up rows.
-          bf16x4 o[2];
+          __bf16* dst = a.y + p * a.plane + (int64_t)m * a.ldy + col;
 #pragma unroll
-          for (int g = 0; g < 2; ++g)
+          for (int gp = 0; gp < 2; ++gp) {
+            const bf16x8 vlo = pair16(lo[2 * gp], lo[2 * gp + 1]);
+            const bf16x8 vhi = pair16(hi[2 * gp], hi[2 * gp + 1]);
+            if (row_ok) {
+              store8(dst + 16 * gp + 8 * h, vlo, 8);
+              store8(dst + 32 + 16 * gp + 8 * h, vhi, 8);
+            }
+          }
+        }
+      } else if constexpr (epi_gated(E)) {
+        // A 32-row block of the packed weight is 16 gate rows then the 16
+        // up rows of the same 16 output columns: registers 4g+e (g = 0, 1)
+        // hold gate rows, 4(g+2)+e the matching up rows.
+        bf16x4 o[2];
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-              o[g][e] = to_bf16(epi_gate<E>(acc[i][j][4 * g + e], acc[i][j][4 * (g + 2) + e]));
-          const bf16x8 v = pair16(o[0], o[1]);
-          put(m, out_n0 + i * 16 + 8 * h, v);
-        } else {
+        for (int g = 0; g < 2; ++g)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            o[g][e] = to_bf16(epi_gate<E>(acc[i][j][4 * g + e], acc[i][j][4 * (g + 2) + e]));
+        const bf16x8 v = pair16(o[0], o[1]);
+        put(m, out_n0 + i * 16 + 8 * h, v);
+      } else {
+#pragma unroll
+        for (int gp = 0; gp < 2; ++gp) {
+          bf16x4 p[2];
+#pragma unroll
+          for (int q = 0; q < 2; ++q)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) p[q][e] = to_bf16(acc[i][j][4 * (2 * gp + q) + e]);
+          bf16x8 v = pair16(p[0], p[1]);
+          const int n = out_n0 + i * 32 + 16 * gp + 8 * h;
+          if constexpr (E != kEpiNone) {
+            bf16x8 b = {}, r = {};
+            if constexpr (kBiasRegs) b = rbias[i][gp];
+            else if constexpr (kPipe && epi_has_bias<E>()) b = cbias[gp];
+            else if constexpr (epi_has_bias<E>()) b = get_bias(n);
+            if constexpr (epi_has_resid<E>()) {
+              if (kResLds && res_in_lds) r = *reinterpret_cast<const bf16x8*>(res_lds + ((m - m0) * BN + (n - n0)) * 2);
+              else if constexpr (kResRegs) r = rres[j][i][gp];
+              else if constexpr (kPipe) r = cres[gp];
+              else r = get_resid(m, n);
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+              float t = epi_pre<E>(to_f32(v[e]), to_f32(b[e]));
+              if constexpr (epi_has_resid<E>()) t = round_bf16(t + to_f32(r[e]));
+              v[e] = to_bf16(t);
+            }
+          }
+          put(m, n, v);
+        }
+      }
+    };
+    if constexpr (!kVec) {
+#pragma unroll
+      for (int j = 0; j < S::FM; ++j) {
+        const int m = m0 + wm * S::TM + j * 32 + frow;
+        const bool row_ok = m < a.M;
+#pragma unroll
+        for (int i = 0; i < S::FN; ++i)
 #pragma unroll
           for (int gp = 0; gp < 2; ++gp) {
             bf16x4 p[2];
@@ -911,26 +954,57 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) /
               for (int e = 0; e < 4; ++e) p[q][e] = to_bf16(acc[i][j][4 * (2 * gp + q) + e]);
             bf16x8 v = pair16(p[0], p[1]);
             const int n = out_n0 + i * 32 + 16 * gp + 8 * h;
-            if constexpr (E != kEpiNone) {
-              bf16x8 b = {}, r = {};
-              if constexpr (kBiasRegs) b = rbias[i][gp];
-              else if constexpr (epi_has_bias<E>()) b = get_bias(n);
-              if constexpr (epi_has_resid<E>()) {
-                if (kResLds && res_in_lds) r = *reinterpret_cast<const bf16x8*>(res_lds + ((m - m0) * BN + (n - n0)) * 2);
-                else if constexpr (kResRegs) r = rres[j][i][gp];
-                else r = get_resid(m, n);
+            if (row_ok && n < a.Nout) {
+              const int valid = a.Nout - n;
+              float b[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+              if constexpr (kBiasRegs) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) b[e] = to_f32(rbias[i][gp][e]);
+              } else if constexpr (epi_has_bias<E>()) {
+                load8(a.bias + n, b, valid);
+              }
+              float r[8];
+              if (kResLds && res_in_lds) {
+                const bf16x8 rv = *reinterpret_cast<const bf16x8*>(res_lds + ((m - m0) * BN + (n - n0)) * 2);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) r[e] = to_f32(rv[e]);
+              } else if constexpr (kResRegs) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) r[e] = to_f32(rres[j][i][gp][e]);
+              } else {
+                load8(a.resid + (int64_t)m * a.ldr + n, r, valid);
               }
 #pragma unroll
-              for (int e = 0; e < 8; ++e) {
-                float t = epi_pre<E>(to_f32(v[e]), to_f32(b[e]));
-                if constexpr (epi_has_resid<E>()) t = round_bf16(t + to_f32(r[e]));
-                v[e] = to_bf16(t);
-              }
+              for (int e = 0; e < 8; ++e) v[e] = to_bf16(round_bf16(epi_pre<E>(to_f32(v[e]), b[e]) + r[e]));
+              store8(a.y + (int64_t)m * a.ldy + n, v, valid);
             }
-            put(m, n, v);
           }
-        }
       }
+    } else if constexpr (kPipe) {
+      // All rows of a column block are read before its first store: one round
+      // trip per column block, not one per 32x32 block (Qwen3.5-small out_proj
+      // and down at 8192 tokens 124 -> 120 and 173 -> 169 us, ModernBERT-large
+      // mlp.Wo there 49.8 -> 46.3).
+#pragma unroll
+      for (int i = 0; i < S::FN; ++i) {
+        bf16x8 cbias[2] = {}, cres[S::FM][2] = {};
+#pragma unroll
+        for (int gp = 0; gp < 2; ++gp) {
+          const int n = out_n0 + i * 32 + 16 * gp + 8 * h;
+          if constexpr (epi_has_bias<E>() && !kBiasRegs) cbias[gp] = get_bias(n);
+          if constexpr (epi_has_resid<E>() && !kResRegs)
+#pragma unroll
+            for (int j = 0; j < S::FM; ++j) cres[j][gp] = get_resid(m0 + wm * S::TM + j * 32 + frow, n);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < S::FM; ++j) block(j, i, cbias, cres[j]);
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < S::FM; ++j)
+#pragma unroll
+        for (int i = 0; i < S::FN; ++i) block(j, i, nullptr, nullptr);
     }
   };
 

@@ -255,10 +255,21 @@ double model_cost(const Context* c, int id, int epi, int64_t M, int64_t N, int64
   const bool lone_pair = occupancy(c, id, epi) >= 2 && grid <= c->cus;
   const double latency = e.pw && grid >= c->cus && !lone_pair ? kProducerLatencyClk : kLatencyClk;
   const double per_kt = std::max(share * std::max(mfma, load), latency / (e.stages - 1));
+  // (A bias that the tile epilogue has no registers to read in a batch -- its
+  // rule: accumulators and bias vectors above half of a wave's registers --
+  // costs half as much again, none of it
+  // hidden by a second workgroup: vision qkv at 8192 / 16384 rows ran 77 / 161 us
+  // on the 256x160 and 128x128 plans, 67 / 133 on the ping-pong shape, which
+  // batches it.)
+  const int waves_per_simd = (e.threads / 64 * e.occupancy + 3) / 4;
+  const int fn = e.tn / 32, blocks = e.streamk ? 0 : e.bm / e.wm / 32 * fn;
+  const bool bias = epi == kEpiBias || epi == kEpiBiasGelu || epi == kEpiBiasResidual || epi == kEpiBiasGeluTanh;
+  const bool bias_reads = bias && e.pw >= 0 && blocks * 16 + fn * 8 > 512 / waves_per_simd / 2;
+  const double epi_cost = epi == kEpiNone ? 1.0 : bias_reads ? 3.0 : 2.0;
   const double store =
       e.streamk ? share * 2.0 * e.bm * e.bn / kStoreBytesPerClk
-                : share * 2.0 * e.bm * e.bn / kTileStoreBytesPerClk * (epi == kEpiNone ? 1.0 : 2.0) *
-                      (occupancy(c, id, epi) >= 2 ? 0.5 : 1.0);
+                : share * 2.0 * e.bm * e.bn / kTileStoreBytesPerClk * epi_cost *
+                      (occupancy(c, id, epi) >= 2 && !bias_reads ? 0.5 : 1.0);
   // The weight stream's floor.  Up to 128 tokens in one tile row,
   // fewer than ~3/4 of the CUs cannot draw the chip's rate: measured on
   // Qwen3.5-27B gate_up at M = 128 (one round of whole tiles), 182 CUs
