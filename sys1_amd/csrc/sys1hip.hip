@@ -53,6 +53,7 @@ struct Plan {
   int64_t grid = 1;
   int64_t dp = 0;  // tiles run whole before the stream phase (stream-K kernels)
   double cost = 1e300;
+  double busy = 1e300;  // the cost without the weight stream's floor
 };
 
 struct PlanKey {
@@ -231,8 +232,9 @@ int occupancy(const Context* c, int id, int epi) {
 // one workgroup per CU against the plain shape at two).
 constexpr double kLowOccupancyRate = 0.7;
 
+// (*busy: the same without the HBM floor.)
 double model_cost(const Context* c, int id, int epi, int64_t M, int64_t N, int64_t K,
-                  int64_t grid, int64_t dp) {
+                  int64_t grid, int64_t dp, double* busy) {
   const KernelEntry& e = kKernels[id];
   const int64_t tiles = cdiv(M, e.bm) * cdiv(N, e.bn);
   const int64_t kts = cdiv(K, e.bk);
@@ -306,6 +308,7 @@ double model_cost(const Context* c, int id, int epi, int64_t M, int64_t N, int64
       t += 2.0 * 2.0 * sg * e.bm * e.bn * 4.0 / kHbmBytesPerClk;  // partial traffic
     }
   }
+  *busy = t;
   return std::max(t, hbm);
 }
 
@@ -360,10 +363,18 @@ void consider(const Context* c, int id, int epi, int64_t M, int64_t N, int64_t K
   }
   for (int64_t dp : cand) {
     if (dp < 0 || (tiles - dp) * (e.threads / 64) > kCounterSlots) continue;
-    const double cost = model_cost(c, id, epi, M, N, K, grid, dp);
+    double busy = 0.0;
+    const double cost = model_cost(c, id, epi, M, N, K, grid, dp, &busy);
     const bool tie = best->kernel >= 0 && cost <= best->cost * 1.001 && cost >= best->cost * 0.999;
-    if (cost < best->cost * 0.999 || (tie && stream_preferred(id, dp, *best, M))) {
-      best->kernel = id, best->grid = grid, best->dp = dp, best->cost = cost;
+    // Two tile plans at the weight stream's floor: the one with less work
+    // under it.  (27B gate_up, the only weight that large, at 129 / 200 / 256
+    // tokens: 89.5 / 95.8 / 105 us on 218 whole 256x160 tiles, 129 / 140 / 156
+    // on 272 256x128 ones, 107-112 on 136 ping-pong ones.)
+    // (Not a taller tile than one that covers M already.)
+    const bool less = tie && !e.streamk && !kKernels[best->kernel].streamk && busy < 0.98 * best->busy &&
+                      !(kKernels[best->kernel].bm >= M && e.bm > kKernels[best->kernel].bm);
+    if (cost < best->cost * 0.999 || less || (tie && stream_preferred(id, dp, *best, M))) {
+      best->kernel = id, best->grid = grid, best->dp = dp, best->cost = cost, best->busy = busy;
     }
   }
 }
