@@ -252,8 +252,9 @@ SYS1HIP_API int sys1hip_linear_rope_qkv_bf16(void* ctx, const uint16_t* x, int64
  *                       (src/archs/qwen35_text.rs:178-203, used at :933,939)
  * Replaces `x.apply(&norm)?.apply(&linear)` at those sites: the norm weight
  * is folded into the projection weight once at load (fold_norm_weight), the
- * call computes per-row statistics of x and then the projection of the raw
- * x with the normalisation applied to the accumulators. */
+ * call computes per-row statistics of x, before the projection or within it,
+ * and the projection of the raw x with the normalisation applied to the
+ * accumulators. */
 #define SYS1HIP_NORM_LAYER 1
 #define SYS1HIP_NORM_RMS 2
 

@@ -27,9 +27,8 @@ enum Epi : int {
   kEpiBiasGelu = 5,
   kEpiBiasResidual = 6,
   kEpiRopeQkv = 7,   // Wqkv: RoPE on q and k, q/k/v written as three planes
-  // Pre-norm projections (the norm's weight folded into w; per-row mean and
-  // reciprocal deviation in `stats`, per-row sums of the folded w in
-  // `colsum`): y = epi(r_m (acc - mu_m c_n)) for LayerNorm, epi(r_m acc) for
+  // Pre-norm projections (the norm's weight folded into w; the row statistics
+  // as GemmArgs::stats says, per-row sums of the folded w in `colsum`): y = epi(r_m (acc - mu_m c_n)) for LayerNorm, epi(r_m acc) for
   // RMSNorm, with epi the base epilogue named.
   kEpiNormLn = 8,
   kEpiNormLnGeglu = 9,

@@ -6,9 +6,10 @@
 //   y[m,n] = sum_k ((x[m,k] - mu_m) r_m g_k) W[n,k]
 //          = r_m (sum_k x[m,k] W'[n,k] - mu_m c_n),   W' = W (.) g,  c_n = sum_k W'[n,k]
 // and an RMSNorm with alpha = 1 + w is y[m,n] = r_m sum_k x[m,k] W'[n,k],
-// W' = W (.) alpha.  The GEMM therefore reads the raw activations; the
-// kernels below supply (mu_m, r_m) per row and W', c at load time, and the
-// GEMM epilogue applies r_m (acc - mu_m c_n).
+// W' = W (.) alpha.  The GEMM therefore reads the raw activations and its
+// epilogue applies r_m (acc - mu_m c_n).  The kernels below supply W', c at
+// load time and, for the tile kernels and the fused conv, (mu_m, r_m) per
+// row; the skinny and stream-K kernels sum each row as they multiply it.
 //   LayerNorm: src/archs/modernbert.rs:1005-1034 (Norm, LayerNorm::new_no_bias;
 //              candle-nn 0.11.0 LayerNorm: mean, then the mean of squared
 //              deviations, r = 1/sqrt(var + eps), all in f32).

@@ -367,9 +367,11 @@ void consider(const Context* c, int id, int epi, int64_t M, int64_t N, int64_t K
     const double cost = model_cost(c, id, epi, M, N, K, grid, dp, &busy);
     const bool tie = best->kernel >= 0 && cost <= best->cost * 1.001 && cost >= best->cost * 0.999;
     // Two tile plans at the weight stream's floor: the one with less work
-    // under it.  (27B gate_up, the only weight that large, at 129 / 200 / 256
-    // tokens: 89.5 / 95.8 / 105 us on 218 whole 256x160 tiles, 129 / 140 / 156
-    // on 272 256x128 ones, 107-112 on 136 ping-pong ones.)
+    // under it.  (27B gate_up, the only weight that large, each kernel forced
+    // in turn at 129 / 200 / 256 tokens: 89.5 / 95.8 / 105 us on 218 whole
+    // 256x160 tiles, 129 / 140 / 156 on 272 256x128 ones, 107-112 on 136
+    // ping-pong ones.  Chosen by this rule it took 107 / 106 us at 200 / 256,
+    // from 138 / 142 on 136 of the earlier 256x256 tiles.)
     // (Not a taller tile than one that covers M already.)
     const bool less = tie && !e.streamk && !kKernels[best->kernel].streamk && busy < 0.98 * best->busy &&
                       !(kKernels[best->kernel].bm >= M && e.bm > kKernels[best->kernel].bm);
