@@ -28,8 +28,9 @@ enum Epi : int {
   kEpiBiasResidual = 6,
   kEpiRopeQkv = 7,   // Wqkv: RoPE on q and k, q/k/v written as three planes
   // Pre-norm projections (the norm's weight folded into w; the row statistics
-  // as GemmArgs::stats says, per-row sums of the folded w in `colsum`): y = epi(r_m (acc - mu_m c_n)) for LayerNorm, epi(r_m acc) for
-  // RMSNorm, with epi the base epilogue named.
+  // as GemmArgs::stats says, per-row sums of the folded w in `colsum`):
+  // y = epi(r_m (acc - mu_m c_n)) for LayerNorm, epi(r_m acc) for RMSNorm,
+  // with epi the base epilogue named.
   kEpiNormLn = 8,
   kEpiNormLnGeglu = 9,
   kEpiNormRms = 10,
@@ -237,11 +238,12 @@ struct GemmArgs {
   const int* pos;
   int rope_rows;        // table rows: positions are clamped into [0, rope_rows)
   int64_t plane;
-  // Pre-norm epilogues: colsum[n] = sum_k w[n, k] (LayerNorm).  The tile
-  // kernels (and every fused conv) read the statistics of a pass before them,
-  // stats[2m] = mean (0 for RMSNorm), stats[2m+1] = 1/sqrt(var + eps); the
-  // skinny and stream-K kernels take each row's sums from the fragments they
-  // multiply (RowSums), with the partial sums of split tiles in `stats`.
+  // Pre-norm epilogues: colsum[n] = sum_k w[n, k] (LayerNorm), and the
+  // statistics of a pass before the launch, stats[2m] = mean (0 for RMSNorm),
+  // stats[2m+1] = 1/sqrt(var + eps).  No such pass where a kernel takes them
+  // itself: LayerNorm's on the skinny kernels where own_layer_stats says so;
+  // RMSNorm's on the skinny and stream-K kernels, from the fragments that
+  // they multiply (RowSums, with the partial sums of split tiles in `stats`).
   float* stats;
   const float* colsum;
   float eps;
@@ -261,82 +263,92 @@ constexpr int kBlkRows = 32;                  // rows of a weight block
 constexpr int kBlkK = 64;                     // k values of a weight block
 constexpr int kBlkBytes = kBlkRows * kBlkK * 2;  // 4 KB
 
-// Sum over the 64 lanes of a wave, the same order on every call.
+// Sum over the 64 lanes of a wave, the same order on every call: lanes 32
+// apart, then 16, 8, 4, 2 and 1 (a value that repeats every 2n lanes is the
+// same n lanes on as n lanes across).  In registers: through LDS (shuffles)
+// the 12 steps of each of 64 rows cost a skinny LayerNorm kernel 1 us more
+// (K = 768, N = 2304 at 100 tokens 10.1 against 9.1).
+template <int DPP>
+__device__ __forceinline__ float add_dpp(float v) {
+  return v + __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), DPP, 0xf, 0xf, true));
+}
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  unsigned u = __builtin_bit_cast(unsigned, v);
+  const auto h = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  u = __builtin_bit_cast(unsigned, __builtin_bit_cast(float, (unsigned)h[0]) + __builtin_bit_cast(float, (unsigned)h[1]));
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  v = __builtin_bit_cast(float, (unsigned)r[0]) + __builtin_bit_cast(float, (unsigned)r[1]);
+  constexpr int kRowRor = 0x120;  // rotate within rows of 16 lanes
+  v = add_dpp<kRowRor + 8>(v);
+  v = add_dpp<kRowRor + 4>(v);
+  v = add_dpp<kRowRor + 2>(v);
+  return add_dpp<kRowRor + 1>(v);
 }
 
-// Pre-norm row statistics taken while a kernel multiplies: the running sum
-// (LayerNorm only) and sum of squares of one lane's share of a row, from the
-// bf16 activation fragments already in registers.  v_dot2_f32_bf16 adds two
-// products exactly formed and rounded in f32: 4 (RMSNorm) or 8 instructions
-// per 16-byte fragment in the shadow of its MFMAs, in place of a launch in
-// front of the projection.  For the latency-bound skinny and stream-K
-// kernels: two ModernBERT-large layers at 64 tokens 68.4 -> 62.5 us, the
-// 27B-width RMSNorm + q|k|v at 8 tokens 38.0 -> 35.6 us.
+// RMSNorm's row statistic taken while a kernel multiplies: the running sum of
+// squares of one lane's share of a row, from the bf16 activation fragments
+// already in registers.  v_dot2_f32_bf16 adds two products exactly formed and
+// rounded in f32: 4 instructions per 16-byte fragment in the shadow of its
+// MFMAs, in place of a launch in front of the projection.  For the
+// latency-bound skinny and stream-K kernels: the 27B-width RMSNorm + q|k|v at
+// 8 tokens 38.0 -> 35.6 us.
 template <int NORM>
 struct RowSums {
-  float s = 0.0f, q = 0.0f;
+  float q = 0.0f;
   __device__ __forceinline__ void add(const i32x4& frag) {
     typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-    const bf16x2_t one = {__bf16(1.0f), __bf16(1.0f)};
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int pair = frag[e];  // (a copy: __builtin_bit_cast of a vector element reads element 0)
       const bf16x2_t v = __builtin_bit_cast(bf16x2_t, pair);
-      if constexpr (NORM == kNormLayer) s = __builtin_amdgcn_fdot2_f32_bf16(v, one, s, false);
-      if constexpr (NORM != kNormNone) q = __builtin_amdgcn_fdot2_f32_bf16(v, v, q, false);
+      if constexpr (NORM == kNormRms) q = __builtin_amdgcn_fdot2_f32_bf16(v, v, q, false);
     }
   }
 };
 
-// Mean and 1/sqrt(var + eps) of a row from its sums.  LayerNorm's variance
-// E[x^2] - mean^2 loses mean^2 / var of its 24 bits to cancellation: a row
-// whose mean^2 exceeds kMaxMeanSq variances (or whose sums are not finite)
-// is `bad` and its variance is taken about the mean, from memory
-// (exact_row_stats), as candle's LayerNorm does.
-constexpr float kMaxMeanSq = 16.0f;
-template <int NORM>
-__device__ __forceinline__ bool row_stats_from_sums(float s, float q, int K, float& mean, float& var) {
-  if constexpr (NORM == kNormLayer) {
-    mean = s / (float)K;
-    var = q / (float)K - mean * mean;
-    return !(mean * mean <= kMaxMeanSq * var);
-  } else {
-    mean = 0.0f;
-    var = q / (float)K;
-    return false;
-  }
-}
-
-// The bad rows of a wave, one after the other by the whole wave: lane L's
-// row is `row0 + L * ldx` for every lane set in `bad` (lane 0 its first row).
-__device__ __forceinline__ void exact_row_stats(unsigned long long bad, const __bf16* x, int64_t ldx, int row0,
-                                                int last_row, int K, int lane, int lane_mask, float& mean, float& var) {
-  while (bad) {
-    const int r = __ffsll(bad) - 1;
-    bad &= bad - 1;
-    const __bf16* row = x + (int64_t)min(row0 + r, last_row) * ldx;
-    float s = 0.0f, d2 = 0.0f;
-    for (int k = lane * 8; k < K; k += 64 * 8) {
-      const bf16x8 v = *reinterpret_cast<const bf16x8*>(row + k);
+// LayerNorm's mean and variance of a row that one wave holds: lane l has the
+// elements c * 512 + 8 l + 0 .. 7 in v[c] (chunks past K are not read).  The
+// variance is taken about the mean, as candle's LayerNorm does: E[x^2] -
+// mean^2 loses mean^2 / var of its 24 bits, and its squares overflow where
+// the deviations' do not.
+template <int CH>
+__device__ __forceinline__ void layer_stats(const bf16x8 (&v)[CH], int K, int lane, float& mean, float& var) {
+  float s = 0.0f;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) s += to_f32(v[e]);
+  for (int c = 0; c < CH; ++c)
+    if (c * 512 + lane * 8 < K) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) s += to_f32(v[c][e]);
     }
-    const float mu = wave_sum(s) / (float)K;
-    for (int k = lane * 8; k < K; k += 64 * 8) {
-      const bf16x8 v = *reinterpret_cast<const bf16x8*>(row + k);
+  mean = wave_sum(s) / (float)K;
+  float d2 = 0.0f;
+#pragma unroll
+  for (int c = 0; c < CH; ++c)
+    if (c * 512 + lane * 8 < K) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const float d = to_f32(v[e]) - mu;
+        const float d = to_f32(v[c][e]) - mean;
         d2 += d * d;
       }
     }
-    const float v2 = wave_sum(d2) / (float)K;
-    if ((lane & lane_mask) == r) mean = mu, var = v2;
-  }
+  var = wave_sum(d2) / (float)K;
+}
+
+// Whether a skinny kernel takes LayerNorm's statistics of its own rows, by
+// layer_stats and so bit for bit those of the pass, instead of having the
+// pass run in front of it.  Every workgroup of a row panel repeats them, so
+// it pays while a wave has few rows, each short enough to hold.  us a call on
+// their own / with the pass, same box: K = 1024, N = 3072 at 1 token (1 row a
+// wave) 4.7 / 6.2, at 64 (2 rows) 7.4 / 9.2, at 129 10.4 / 12.2, at 256 (8
+// rows) 12.4 / 12.6; gated N = 5248 at 64 (4 rows) 11.3 / 11.9; K = 768, gated
+// N = 2304 at 400 (8 rows) 13.5 / 13.8.  (Sums of x and x^2 over the fragments
+// took 5.2, 7.6, 10.9, 11.4, 10.7 and 12.7, but a row far off zero then needs
+// its variance again, from memory: 19, 38, 42, 73, 71 and 74 us.)
+constexpr int kOwnStatsRows = 8;                    // rows a wave
+constexpr int kOwnStatsChunks = 2;                  // of 512 elements
+constexpr int kOwnStatsK = kOwnStatsChunks * 512;
+constexpr bool own_layer_stats(int bm, int waves, int64_t K) {
+  return bm <= kOwnStatsRows * waves && K <= kOwnStatsK;
 }
 
 // Map the hardware workgroup id to a logical tile id so that each XCD gets a

@@ -247,13 +247,15 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) /
                            (S::kLdsBytes + BM * BN * 2) * OCC <= 160 * 1024 && (BM * BN * 2 / 1024) % PW == 0;
   constexpr int kResBytes = kResLds ? BM * BN * 2 : 0;
   // Row statistics of a fused pre-norm: under stream-K each compute wave sums
-  // the rows it multiplies (RowSums); the tile kernels read those of a pass
-  // before them.  They were built with sums of their own, both ways, and lost
+  // the squares of the rows it multiplies for RMSNorm (RowSums); the others
+  // read those of a pass before them: LayerNorm's variance is taken about the
+  // mean, which no sum over one walk of K gives (layer_stats).  The tile
+  // kernels were built with sums of their own, both ways, and lost
   // what the pass costs: in the producer waves, from the landed stages, the
   // sums delayed the refills (ModernBERT-base Wi+LN at 8109 tokens 48.9 us
   // against 49.3 with the pass, Qwen3.5-small in_proj at 8192 409.6 against
   // 378.5); in the compute waves they spilled (58.0 and 459.4 us).
-  constexpr bool kStatPass = !STREAMK || epi_base(EPI) == kEpiConvSilu;
+  constexpr bool kStatPass = !STREAMK || epi_base(EPI) == kEpiConvSilu || epi_norm(EPI) == kNormLayer;
   constexpr int kOwnNorm = kStatPass ? kNormNone : epi_norm(EPI);
   // (the ping-pong ring: STAGES_ slots of half the x or half the w rows)
   constexpr int kSlotBytes = (BM > BN ? BM : BN) / 2 * S::kRowBytes;
@@ -577,11 +579,8 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) /
         rs[j] = a.stats[2 * (int64_t)m + 1];
       } else {
         // both halves of the row's k-chunks
-        const float s = sums[j].s + __shfl_xor(sums[j].s, 32, 64), q = sums[j].q + __shfl_xor(sums[j].q, 32, 64);
-        float var;
-        const bool bad = row_stats_from_sums<kOwnNorm>(s, q, a.K, mu[j], var);
-        if constexpr (kOwnNorm == kNormLayer)
-          exact_row_stats(__ballot(bad) & 0xffffffffull, a.x, a.ldx, row0, a.M - 1, a.K, lane, 31, mu[j], var);
+        const float var = (sums[j].q + __shfl_xor(sums[j].q, 32, 64)) / (float)a.K;
+        mu[j] = 0.0f;
         rs[j] = 1.0f / sqrtf(var + a.eps);
       }
     }
@@ -1025,10 +1024,10 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) /
     return (unsigned)((((int64_t)g * 2 + slot) * kTileF4 + wave * kWaveF4 + lane) * 16);
   };
   // The row sums of a fused pre-norm go the same way, to a.stats:
-  // [workgroup][slot][wave][block j][64 lanes] of (sum, sum of squares).
+  // [workgroup][slot][wave][block j][64 lanes].
   const rsrc_t ssr = make_rsrc(a.stats);
   auto sums_off = [&](int g, int slot) -> unsigned {
-    return (unsigned)(((((int64_t)g * 2 + slot) * S::kWaves + wave) * S::FM * 64 + lane) * 8);
+    return (unsigned)(((((int64_t)g * 2 + slot) * S::kWaves + wave) * S::FM * 64 + lane) * 4);
   };
   // A partial segment: write this workgroup's partial; returns true when it
   // is the tile's last segment to arrive, with acc then holding the full sum
@@ -1057,9 +1056,8 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) /
     if constexpr (kOwnNorm != kNormNone) {
 #pragma unroll
       for (int j = 0; j < S::FM; ++j)
-        __builtin_amdgcn_raw_buffer_store_b64(
-            (i32x2){__builtin_bit_cast(int, sums[j].s), __builtin_bit_cast(int, sums[j].q)}, ssr,
-            (int)(sums_off(blockIdx.x, slot) + j * 64 * 8), 0, kCoherent);
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, sums[j].q), ssr,
+                                              (int)(sums_off(blockIdx.x, slot) + j * 64 * 4), 0, kCoherent);
     }
     int g_lo, g_hi;
     walk.tile_owners(t, g_lo, g_hi);
@@ -1082,13 +1080,9 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) /
       const unsigned src = slot_off(g, gslot);
       if constexpr (kOwnNorm != kNormNone) {
 #pragma unroll
-        for (int j = 0; j < S::FM; ++j) {
-          typedef float f32x2_t __attribute__((ext_vector_type(2)));
-          const f32x2_t v = __builtin_bit_cast(
-              f32x2_t, __builtin_amdgcn_raw_buffer_load_b64(ssr, (int)(sums_off(g, gslot) + j * 64 * 8), 0, kCoherent));
-          sums[j].s += v[0];
-          sums[j].q += v[1];
-        }
+        for (int j = 0; j < S::FM; ++j)
+          sums[j].q += __builtin_bit_cast(
+              float, __builtin_amdgcn_raw_buffer_load_b32(ssr, (int)(sums_off(g, gslot) + j * 64 * 4), 0, kCoherent));
       }
       // All of one owner's loads are in flight together (these coherent
       // reads come from beyond the L2: one round trip per owner, not one

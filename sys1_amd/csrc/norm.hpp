@@ -8,8 +8,8 @@
 // and an RMSNorm with alpha = 1 + w is y[m,n] = r_m sum_k x[m,k] W'[n,k],
 // W' = W (.) alpha.  The GEMM therefore reads the raw activations and its
 // epilogue applies r_m (acc - mu_m c_n).  The kernels below supply W', c at
-// load time and, for the tile kernels and the fused conv, (mu_m, r_m) per
-// row; the skinny and stream-K kernels sum each row as they multiply it.
+// load time and (mu_m, r_m) per row, the latter where the projection's kernel
+// does not take them itself (GemmArgs::stats).
 //   LayerNorm: src/archs/modernbert.rs:1005-1034 (Norm, LayerNorm::new_no_bias;
 //              candle-nn 0.11.0 LayerNorm: mean, then the mean of squared
 //              deviations, r = 1/sqrt(var + eps), all in f32).
@@ -43,32 +43,20 @@ __global__ __launch_bounds__(256) void row_stats_kernel(const __bf16* __restrict
       const int k = c * 512 + lane * 8;
       if (k < K) v[c] = *reinterpret_cast<const bf16x8*>(row + k);
     }
-    float s = 0.0f;
-#pragma unroll
-    for (int c = 0; c < kRowChunks; ++c)
-      if (c * 512 + lane * 8 < K) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float f = to_f32(v[c][e]);
-          s += NORM == kNormLayer ? f : f * f;
-        }
-      }
-    s = wave_sum(s);
     if constexpr (NORM == kNormLayer) {
-      mean = s / (float)K;
-      float d2 = 0.0f;
+      layer_stats<kRowChunks>(v, K, lane, mean, var);
+    } else {
+      float s = 0.0f;
 #pragma unroll
       for (int c = 0; c < kRowChunks; ++c)
         if (c * 512 + lane * 8 < K) {
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
-            const float d = to_f32(v[c][e]) - mean;
-            d2 += d * d;
+            const float f = to_f32(v[c][e]);
+            s += f * f;
           }
         }
-      var = wave_sum(d2) / (float)K;
-    } else {
-      var = s / (float)K;
+      var = wave_sum(s) / (float)K;
     }
   } else {
     float s = 0.0f;

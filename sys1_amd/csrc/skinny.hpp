@@ -170,7 +170,7 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs a) {
     for (int u = 0; u < U; ++u) {
       const int st = s + u;
       const bool ok = st < s1 && st * 32 + q * 8 < a.K;
-      const int sc = min(st, s1 - 1);
+      const int sc = max(min(st, s1 - 1), 0);
       const int so = __builtin_amdgcn_readfirstlane(sc * 64);
       const int sw = __builtin_amdgcn_readfirstlane(wstep(sc));
 #pragma unroll
@@ -181,7 +181,7 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs a) {
         bx[b][u][j] = __builtin_amdgcn_raw_buffer_load_b128(xr, ok ? (int)xo[j] : (int)kOutOfRange, so, 0);
     }
   };
-  // Row sums of a fused pre-norm, over this lane's k-chunks of its rows
+  // Row sums of a fused RMSNorm, over this lane's k-chunks of its rows
   // (chunks past K and k-steps past the range are zeros).
   RowSums<NORM> sums[FM];
   auto compute = [&](int b) {
@@ -195,8 +195,55 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs a) {
           if (i == 0) sums[j].add(bx[b][u][j]);
         }
   };
+  // LayerNorm's statistics, into two pad columns of wave 0's slab: those of
+  // the pass, or of the wave's own rows, loaded in front of the k-loop's first
+  // loads and finished behind them (rows past M repeat the last).  All in one
+  // block, own rows masked off where the pass ran and the k-loop's first loads
+  // issued for an empty range too (their offsets are all out of range): with
+  // branches the rows were waited for together with those loads, 8.9 us for
+  // 8.1 at K = 1024, N = 3072, 64 tokens.
+  constexpr bool kOwnStats = NORM == kNormLayer && own_layer_stats(BM, NW, 0);
+  const bool own_stats = kOwnStats && own_layer_stats(BM, NW, a.K);
+  const bool pass_row = NORM == kNormLayer && !own_stats && (int)threadIdx.x < BM;
+  constexpr int kRows = kOwnStats ? BM / NW : 1;
+  const int own_k = own_stats ? a.K : 0;
+  bf16x8 v[kRows][kOwnStatsChunks];
+  if constexpr (kOwnStats) {
+#pragma unroll
+    for (int i = 0; i < kRows; ++i) {
+      const __bf16* row = a.x + (int64_t)min(m0 + wave * kRows + i, a.M - 1) * a.ldx;
+#pragma unroll
+      for (int c = 0; c < kOwnStatsChunks; ++c) {
+        const int k = c * 512 + lane * 8;
+        if (k < own_k) v[i][c] = *reinterpret_cast<const bf16x8*>(row + k);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  float mean_pre = 0.0f, rs_pre = 0.0f;
+  if (pass_row) {
+    const int64_t m = min(m0 + (int)threadIdx.x, a.M - 1);
+    mean_pre = a.stats[2 * m];
+    rs_pre = a.stats[2 * m + 1];
+  }
+  load(0, s0);
+  if constexpr (kOwnStats) {
+    __builtin_amdgcn_sched_barrier(0);
+    if (own_stats) {
+#pragma unroll
+      for (int i = 0; i < kRows; ++i) {
+        float mean, var;
+        layer_stats<kOwnStatsChunks>(v[i], a.K, lane, mean, var);
+        if (lane == 0) {
+          float* st = red + (wave * kRows + i) * S::kRowF32 + BN;
+          st[2] = mean;
+          st[3] = 1.0f / sqrtf(var + a.eps);
+        }
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
   if (s0 < s1) {
-    load(0, s0);
     int s = s0;
     for (; s + U < s1; s += 2 * U) {
       load(1, s + U);
@@ -215,41 +262,32 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs a) {
 #pragma unroll
     for (int j = 0; j < FM; ++j)
       *reinterpret_cast<f32x4*>(mine + (j * 16 + r16) * S::kRowF32 + i * 16 + 4 * q) = acc[i][j];
-  if constexpr (NORM != kNormNone) {
-    // ... and its row sums, over the four lanes of a row, to the two pad
-    // columns at BN.
+  if (pass_row) {
+    red[threadIdx.x * S::kRowF32 + BN + 2] = mean_pre;
+    red[threadIdx.x * S::kRowF32 + BN + 3] = rs_pre;
+  }
+  if constexpr (NORM == kNormRms) {
+    // ... and its row sums, over the four lanes of a row, to the pad column
+    // at BN.
 #pragma unroll
     for (int j = 0; j < FM; ++j) {
-      float s = sums[j].s, qq = sums[j].q;
-      s += __shfl_xor(s, 16, 64);
+      float qq = sums[j].q;
       qq += __shfl_xor(qq, 16, 64);
-      s += __shfl_xor(s, 32, 64);
       qq += __shfl_xor(qq, 32, 64);
-      if (q == 0) {
-        mine[(j * 16 + r16) * S::kRowF32 + BN] = s;
-        mine[(j * 16 + r16) * S::kRowF32 + BN + 1] = qq;
-      }
+      if (q == 0) mine[(j * 16 + r16) * S::kRowF32 + BN] = qq;
     }
   }
   __syncthreads();
-  if constexpr (NORM != kNormNone) {
-    // The first BM threads finish a row's statistics each, into the other
-    // two pad columns of wave 0's slab.
-    if (wave * 64 < BM) {
-      const int r = min((int)threadIdx.x, BM - 1);
-      float s = 0.0f, qq = 0.0f, mean, var;
+  if constexpr (NORM == kNormRms) {
+    // The first BM threads finish a row's statistics each, into the two
+    // statistics columns of wave 0's slab.
+    if ((int)threadIdx.x < BM) {
+      const int r = threadIdx.x;
+      float qq = 0.0f;
 #pragma unroll
-      for (int ww = 0; ww < NW; ++ww) {
-        s += red[(ww * BM + r) * S::kRowF32 + BN];
-        qq += red[(ww * BM + r) * S::kRowF32 + BN + 1];
-      }
-      const bool bad = row_stats_from_sums<NORM>(s, qq, a.K, mean, var) && (int)threadIdx.x < BM;
-      if constexpr (NORM == kNormLayer)
-        exact_row_stats(__ballot(bad), a.x, a.ldx, m0 + wave * 64, a.M - 1, a.K, lane, 63, mean, var);
-      if ((int)threadIdx.x < BM) {
-        red[r * S::kRowF32 + BN + 2] = mean;
-        red[r * S::kRowF32 + BN + 3] = 1.0f / sqrtf(var + a.eps);
-      }
+      for (int ww = 0; ww < NW; ++ww) qq += red[(ww * BM + r) * S::kRowF32 + BN];
+      red[r * S::kRowF32 + BN + 2] = 0.0f;
+      red[r * S::kRowF32 + BN + 3] = 1.0f / sqrtf(qq / (float)a.K + a.eps);
     }
     __syncthreads();
   }

@@ -85,8 +85,9 @@ struct Context {
   float* ws = nullptr;
   unsigned* counters = nullptr;
   // Pre-norm row statistics of the pass, kNormRows x (mean, 1/std), or the
-  // partial row sums of a stream-K call: 8 bytes per row and wave column of
-  // each partial tile, at most 1/16 of the partials' bytes (4 MB of these 8).
+  // partial row sums of a stream-K RMSNorm call: 4 bytes per lane and row
+  // block of each partial tile, at most 1/32 of the partials' bytes (2 MB of
+  // these 8).
   float* stats = nullptr;
   // Projection chains: the dependency bank (zero between launches: each
   // launch's last workgroup clears it) and the error word, one allocation.
@@ -172,9 +173,11 @@ int epi_id_from_flags(int32_t f) {
 int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // Whether a pre-norm projection on kernel `e` reads the row statistics of a
-// pass in front of it (the tile kernels); the skinny and stream-K kernels
-// take them themselves.
-bool needs_stats_pass(const KernelEntry& e) { return !e.skinny && !e.streamk; }
+// pass in front of it, or takes them itself (see GemmArgs::stats).
+bool needs_stats_pass(const KernelEntry& e, int32_t norm, int64_t K) {
+  if (norm == SYS1HIP_NORM_LAYER) return !(e.skinny && own_layer_stats(e.bm, e.threads / 64, K));
+  return !e.skinny && !e.streamk;
+}
 
 // Modelled time (in CU clocks) of a projection on kernel `e` launched on
 // `grid` workgroups, of which the first `dp` tiles run whole (tile phase)
@@ -1131,7 +1134,7 @@ int sys1hip_norm_linear_bf16(void* ctx, const uint16_t* x, int64_t ldx, const ui
   const KernelEntry& e = kKernels[p.kernel];
   if (e.streamk && (cdiv(M, e.bm) * cdiv(N, e.bn) - p.dp) * (e.threads / 64) > kCounterSlots)
     return fail(SYS1HIP_ERANGE, "sys1hip_norm_linear_bf16: more split tiles than stream-K counters");
-  if (needs_stats_pass(e)) {
+  if (needs_stats_pass(e, norm, K)) {
     rc = launch_row_stats(c, reinterpret_cast<const __bf16*>(x), ldx, M, K, norm, eps);
     if (rc) return rc;
   }
@@ -1215,7 +1218,7 @@ int sys1hip_linear_conv_silu_bf16(void* ctx, const uint16_t* x, int64_t ldx, con
   if (e.streamk && (cdiv(rows, e.bm) * cdiv(N, e.bn) - p.dp) * (e.threads / 64) > kCounterSlots)
     return fail(SYS1HIP_ERANGE, "sys1hip_linear_conv_silu_bf16: more split tiles than stream-K counters");
   a.eps = eps;
-  if (norm && (fused || needs_stats_pass(e))) {
+  if (norm && (fused || needs_stats_pass(e, norm, K))) {
     rc = launch_row_stats(c, xb, ldx, M, K, norm, eps);
     if (rc) return rc;
   }

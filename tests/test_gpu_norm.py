@@ -234,11 +234,10 @@ def test_blocked_weight_with_every_norm_epilogue_is_bitwise_row_major(dev, orc):
                                        ("stream_64x256_s4_w2x4_p4", 3)])
 @pytest.mark.parametrize("kind", ["layer", "rms"])
 def test_row_sums_of_the_multiplying_kernels(dev, orc, name, grid, kind):
-    """The skinny and stream-K kernels take the row statistics from their own
-    fragments: rows on both sides of the mean^2 = 16 var line beyond which a
-    variance is taken about the mean (rows 6 and 16 deviations off zero, a
-    ragged last tile row, split tiles), and a row with an infinity, which
-    stays that row's alone.  Projection tolerance, as everywhere."""
+    """The skinny and stream-K kernels on rows up to 16 deviations off zero (a
+    ragged last tile row, split tiles), and with an infinity in a row, which
+    stays that row's alone.  Projection tolerance, as everywhere: the
+    statistics themselves are test_row_statistics_on_every_kernel's."""
     from sys1_amd import kernel_names
     from sys1_amd.norm import NormLinear
     N, K = 330, 712
@@ -266,3 +265,60 @@ def test_row_sums_of_the_multiplying_kernels(dev, orc, name, grid, kind):
     finally:
         dev.set_kernel(-1)
         dev.set_grid(0)
+
+
+def _readout(orc, M, N, K, kind, seed):
+    """Inputs whose products and sums are exact in f32 in any order, so that
+    an output shows its row's statistics and nothing else: small integers
+    around an offset, a power of two per row, and weight rows with one entry
+    (RMSNorm) or a +v, -v pair, whose column sum is zero (LayerNorm)."""
+    rng = np.random.default_rng(seed)
+    rows = [(0, 1.0), (3, 1.0), (50, 2.0 ** -60), (-100, 1.0), (0, 2.0 ** -12), (120, 2.0 ** 40)]
+    if kind == "layer":
+        # sigma 4.9 at 130 * 2^52: the squares' sum overflows f32, the deviations' does not
+        rows.append((120, 2.0 ** 53))
+    off, scale = (np.array(v, np.float64)[np.arange(M) % len(rows)][:, None] for v in zip(*rows))
+    x = (rng.integers(-8, 9, (M, K)) + off) * scale
+    w = np.zeros((N, K), np.float32)
+    v = orc.round_bf16(rng.uniform(0.5, 2.0, N).astype(np.float32))
+    cols = np.stack([rng.permutation(K)[:2] for _ in range(N)])
+    w[np.arange(N), cols[:, 0]] = v
+    if kind == "layer":
+        w[np.arange(N), cols[:, 1]] = -v
+    return x.astype(np.float32), w
+
+
+@pytest.mark.parametrize("kind", ["layer", "rms"])
+@pytest.mark.parametrize("K", [712, 1032])
+def test_row_statistics_on_every_kernel(dev, orc, kind, K):
+    """Whoever takes the row statistics (the pass, a skinny kernel's waves for
+    LayerNorm up to K = 1024, the sums of the skinny and stream-K kernels for
+    RMSNorm): the same outputs bit for bit, each within one bf16 rounding
+    (2^-8) of float64, for rows far off zero, scaled down to where eps is
+    all, and up to where x^2 summed over the row would overflow."""
+    from sys1_amd import kernel_names
+    from sys1_amd.norm import NormLinear
+    N, eps = 200, 1e-5
+    names = kernel_names()
+    first = names.index("tile_128x128_s2_w2x2")
+    order = [first] + [i for i in range(len(names)) if i != first]
+    try:
+        for M in (1, 17, 133, 300):
+            x, w = _readout(orc, M, N, K, kind, 7 * M + K)
+            x64 = x.astype(np.float64)
+            mu = x64.mean(1, keepdims=True) if kind == "layer" else 0.0
+            # (a LayerNorm's mean term drops out: the weight rows sum to zero)
+            ref = x64 @ w.T.astype(np.float64) / np.sqrt(((x64 - mu) ** 2).mean(1, keepdims=True) + eps)
+            g = torch.ones(K) if kind == "layer" else torch.zeros(K)
+            lin = NormLinear(to_gpu_bf16(w, torch), g, kind, eps, None, device=dev)
+            xg = to_gpu_bf16(x, torch)
+            for kid in order:
+                dev.set_kernel(kid)
+                print(f"[gpu] statistics {names[kid]} {kind} M={M} K={K}", flush=True)
+                y = to_np(lin(xg))
+                if kid == first:
+                    expect = y
+                    assert (np.abs(y - ref) <= 2.0 ** -8 * np.abs(ref)).all()
+                np.testing.assert_array_equal(y, expect, err_msg=f"{names[kid]} M={M}")
+    finally:
+        dev.set_kernel(-1)
