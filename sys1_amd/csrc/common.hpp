@@ -291,17 +291,24 @@ __device__ __forceinline__ float wave_sum(float v) {
 // rounded in f32: 4 instructions per 16-byte fragment in the shadow of its
 // MFMAs, in place of a launch in front of the projection.  For the
 // latency-bound skinny and stream-K kernels: the 27B-width RMSNorm + q|k|v at
-// 8 tokens 38.0 -> 35.6 us.
+// 8 tokens 37.8 -> 35.5 us.  The fragments' sums are added up in f64: in f32 a
+// stream-K lane's chain of K / 4 additions lost 3 to 7 times what the pass's
+// K / 64 do (emulated, 400 rows, root mean square: 3.8e-7 of the sum against
+// 0.9e-7 at K = 5120, 2.3e-6 against 4.1e-7 at 17408; so 0.3e-7 at both).
 template <int NORM>
 struct RowSums {
-  float q = 0.0f;
+  double q = 0.0;
   __device__ __forceinline__ void add(const i32x4& frag) {
     typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+    if constexpr (NORM == kNormRms) {
+      float f = 0.0f;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int pair = frag[e];  // (a copy: __builtin_bit_cast of a vector element reads element 0)
-      const bf16x2_t v = __builtin_bit_cast(bf16x2_t, pair);
-      if constexpr (NORM == kNormRms) q = __builtin_amdgcn_fdot2_f32_bf16(v, v, q, false);
+      for (int e = 0; e < 4; ++e) {
+        const int pair = frag[e];  // (a copy: __builtin_bit_cast of a vector element reads element 0)
+        const bf16x2_t v = __builtin_bit_cast(bf16x2_t, pair);
+        f = __builtin_amdgcn_fdot2_f32_bf16(v, v, f, false);
+      }
+      q += (double)f;
     }
   }
 };

@@ -579,7 +579,7 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) /
         rs[j] = a.stats[2 * (int64_t)m + 1];
       } else {
         // both halves of the row's k-chunks
-        const float var = (sums[j].q + __shfl_xor(sums[j].q, 32, 64)) / (float)a.K;
+        const float var = (float)((sums[j].q + __shfl_xor(sums[j].q, 32, 64)) / a.K);
         mu[j] = 0.0f;
         rs[j] = 1.0f / sqrtf(var + a.eps);
       }
@@ -1027,7 +1027,7 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) /
   // [workgroup][slot][wave][block j][64 lanes].
   const rsrc_t ssr = make_rsrc(a.stats);
   auto sums_off = [&](int g, int slot) -> unsigned {
-    return (unsigned)(((((int64_t)g * 2 + slot) * S::kWaves + wave) * S::FM * 64 + lane) * 4);
+    return (unsigned)(((((int64_t)g * 2 + slot) * S::kWaves + wave) * S::FM * 64 + lane) * 8);
   };
   // A partial segment: write this workgroup's partial; returns true when it
   // is the tile's last segment to arrive, with acc then holding the full sum
@@ -1056,8 +1056,8 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) /
     if constexpr (kOwnNorm != kNormNone) {
 #pragma unroll
       for (int j = 0; j < S::FM; ++j)
-        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, sums[j].q), ssr,
-                                              (int)(sums_off(blockIdx.x, slot) + j * 64 * 4), 0, kCoherent);
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(i32x2, sums[j].q), ssr,
+                                              (int)(sums_off(blockIdx.x, slot) + j * 64 * 8), 0, kCoherent);
     }
     int g_lo, g_hi;
     walk.tile_owners(t, g_lo, g_hi);
@@ -1082,7 +1082,7 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) /
 #pragma unroll
         for (int j = 0; j < S::FM; ++j)
           sums[j].q += __builtin_bit_cast(
-              float, __builtin_amdgcn_raw_buffer_load_b32(ssr, (int)(sums_off(g, gslot) + j * 64 * 4), 0, kCoherent));
+              double, __builtin_amdgcn_raw_buffer_load_b64(ssr, (int)(sums_off(g, gslot) + j * 64 * 8), 0, kCoherent));
       }
       // All of one owner's loads are in flight together (these coherent
       // reads come from beyond the L2: one round trip per owner, not one

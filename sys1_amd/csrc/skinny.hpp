@@ -267,14 +267,14 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs a) {
     red[threadIdx.x * S::kRowF32 + BN + 3] = rs_pre;
   }
   if constexpr (NORM == kNormRms) {
-    // ... and its row sums, over the four lanes of a row, to the pad column
-    // at BN.
+    // ... and its row sums, over the four lanes of a row, to the two pad
+    // columns at BN (8-byte aligned: BN and kRowF32 are even).
 #pragma unroll
     for (int j = 0; j < FM; ++j) {
-      float qq = sums[j].q;
+      double qq = sums[j].q;
       qq += __shfl_xor(qq, 16, 64);
       qq += __shfl_xor(qq, 32, 64);
-      if (q == 0) mine[(j * 16 + r16) * S::kRowF32 + BN] = qq;
+      if (q == 0) *reinterpret_cast<double*>(mine + (j * 16 + r16) * S::kRowF32 + BN) = qq;
     }
   }
   __syncthreads();
@@ -283,11 +283,11 @@ __global__ __launch_bounds__(NW * 64) void skinny_kernel(GemmArgs a) {
     // statistics columns of wave 0's slab.
     if ((int)threadIdx.x < BM) {
       const int r = threadIdx.x;
-      float qq = 0.0f;
+      double qq = 0.0;
 #pragma unroll
-      for (int ww = 0; ww < NW; ++ww) qq += red[(ww * BM + r) * S::kRowF32 + BN];
+      for (int ww = 0; ww < NW; ++ww) qq += *reinterpret_cast<const double*>(red + (ww * BM + r) * S::kRowF32 + BN);
       red[r * S::kRowF32 + BN + 2] = 0.0f;
-      red[r * S::kRowF32 + BN + 3] = 1.0f / sqrtf(qq / (float)a.K + a.eps);
+      red[r * S::kRowF32 + BN + 3] = 1.0f / sqrtf((float)(qq / a.K) + a.eps);
     }
     __syncthreads();
   }

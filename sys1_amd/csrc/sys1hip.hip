@@ -85,8 +85,8 @@ struct Context {
   float* ws = nullptr;
   unsigned* counters = nullptr;
   // Pre-norm row statistics of the pass, kNormRows x (mean, 1/std), or the
-  // partial row sums of a stream-K RMSNorm call: 4 bytes per lane and row
-  // block of each partial tile, at most 1/32 of the partials' bytes (2 MB of
+  // partial row sums of a stream-K RMSNorm call: 8 bytes per lane and row
+  // block of each partial tile, at most 1/16 of the partials' bytes (4 MB of
   // these 8).
   float* stats = nullptr;
   // Projection chains: the dependency bank (zero between launches: each

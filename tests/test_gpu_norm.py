@@ -322,3 +322,45 @@ def test_row_statistics_on_every_kernel(dev, orc, kind, K):
                 np.testing.assert_array_equal(y, expect, err_msg=f"{names[kid]} M={M}")
     finally:
         dev.set_kernel(-1)
+
+
+@pytest.mark.parametrize("grid", [0, 7])
+def test_rms_row_sums_hold_their_precision(dev, orc, grid):
+    """The sums of squares that the skinny and stream-K kernels take: a row of
+    ones behind one 2^13, whose square an f32 sum would add no 1 or 2 to (a
+    lane's whole share lost: f32 sums were up to 4.8e-6 of 1/rms off).  Read
+    off 1/rms to 2^-21 from the column whose product first rounds to bf16's
+    1 + 2^-7; bound 1e-6: 3 of the 2^13's fragment's 4 f32 sums round by up to
+    4 (0.9e-7 of 1/rms), the mean, root, quotient and product 0.6e-7 each at
+    most, the column 4.8e-7."""
+    from sys1_amd import kernel_names
+    from sys1_amd.norm import NormLinear
+    N, K, M = 512, 5120, 40
+    x = np.ones((M, K), np.float32)
+    x[np.arange(M), (np.arange(M) * 136) % (K - 8)] = 2.0 ** 13  # (row 0: its first element)
+    r = 1.0 / np.sqrt((x.astype(np.float64) ** 2).mean(1)[0] + 1e-6)  # the same for every row
+    # products v_n around (1 + 2^-8) / r, 2^-21 apart, as three bf16 parts on columns where x = 1
+    v = ((1 + 2.0 ** -8) / r * (1 + (np.arange(N) - N // 2) * 2.0 ** -21)).astype(np.float32)
+    w = np.zeros((N, K), np.float32)
+    rest = v.copy()
+    for c in (K - 7, K - 4, K - 1):
+        w[:, c] = orc.round_bf16(rest)
+        rest = rest - w[:, c]
+    assert (rest == 0).all() and (x[:, [K - 7, K - 4, K - 1]] == 1).all()
+    lin = NormLinear(to_gpu_bf16(w, torch), torch.zeros(K), "rms", 1e-6, None, device=dev)
+    xg = to_gpu_bf16(x, torch)
+    try:
+        dev.set_grid(grid)
+        for kid, name in enumerate(kernel_names()):
+            if not name.startswith(("skinny_", "stream_")):
+                continue
+            dev.set_kernel(kid)
+            print(f"[gpu] rms row sums {name} grid={grid}", flush=True)
+            y = to_np(lin(xg))
+            assert np.isin(y, [1.0, 1.0 + 2.0 ** -7]).all()
+            first = (y > 1.0).argmax(axis=1)
+            err = -(first - N // 2) * 2.0 ** -21
+            assert np.abs(err).max() <= 1e-6, f"{name}: {np.abs(err).max():.1e}"
+    finally:
+        dev.set_kernel(-1)
+        dev.set_grid(0)
