@@ -758,9 +758,9 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) /
     // test and a divergent branch per 16 bytes (the vision tower's fc1 at 3001
     // rows 43.7 -> 39.8 us, 27B gate_up at 4096 tokens 1162 -> 1128, where the
     // ping-pong groups' epilogues follow each other; 256x160 plans 0-2%).
-    // (Not for bias and residual together at three waves per SIMD, whose
-    // descriptors spill into the k-loop: vision fc2 on 256x160 104 -> 112 us.
-    // Nor beside the residual's LDS copy: 15 registers spill, not 4.)
+    // (At three and four waves per SIMD not for bias and residual together,
+    // whose descriptors spill into the k-loop: vision fc2 on 256x160 104 ->
+    // 112 us.  Nor beside the residual's LDS copy: 15 registers spill, not 4.)
     constexpr bool kVec = kWavesPerSimd <= 2 || !(E == kEpiBiasResidual || kResLds);
     const bool vec_n = kVec && a.Nout % 8 == 0;
     const bool vec_y = vec_n && a.ldy % 8 == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0 &&
@@ -992,8 +992,9 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) /
           const int n = out_n0 + i * 32 + 16 * gp + 8 * h;
           if constexpr (epi_has_bias<E>() && !kBiasRegs) cbias[gp] = get_bias(n);
           if constexpr (epi_has_resid<E>() && !kResRegs)
+            if (!(kResLds && res_in_lds))  // (block() takes it from the LDS copy)
 #pragma unroll
-            for (int j = 0; j < S::FM; ++j) cres[j][gp] = get_resid(m0 + wm * S::TM + j * 32 + frow, n);
+              for (int j = 0; j < S::FM; ++j) cres[j][gp] = get_resid(m0 + wm * S::TM + j * 32 + frow, n);
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll

@@ -609,7 +609,8 @@ def test_ping_pong_tiles_at_their_edges(dev, orc, M, N, K, grid, blocked):
         dev.set_grid(0)
 
 
-@pytest.mark.parametrize("name", ["tile_128x192_s3_w4x2_p4", "tile_256x256_s10_w2x4_pp", "stream_64x256_s4_w2x4_p4"])
+@pytest.mark.parametrize("name", ["tile_128x192_s3_w4x2_p4", "tile_256x256_s10_w2x4_pp", "stream_64x256_s4_w2x4_p4",
+                                  "tile_128x160_s3_w4x1_p4", "tile_128x96_s2_w4x1_p4"])
 @pytest.mark.parametrize("M,N,ld,off", [
     (3, 200, 200, 0),            # every row 16-byte aligned
     (130, 200, 208, 8),          # a column slice, aligned
@@ -619,9 +620,10 @@ def test_ping_pong_tiles_at_their_edges(dev, orc, M, N, K, grid, blocked):
     (2, 200, 1 << 29, 0),        # row offsets past 32 bits: a tile row 4 would wrap onto row 0
 ])
 def test_epilogue_addressing(dev, orc, name, M, N, ld, off):
-    """The epilogue's buffer-addressed outputs and residuals and the checked
-    element-wise ones: in place over a strided view, nothing outside it
-    touched, each output within one bf16 ulp of the rounded sum."""
+    """The epilogue's buffer-addressed outputs and residuals, the checked
+    element-wise ones and the residual's LDS copy (the last two names): in
+    place over a strided view, nothing outside it touched, each output within
+    one bf16 ulp of the rounded sum."""
     from sys1_amd import kernel_names
     from sys1_amd.linear import Linear
     K = 128
