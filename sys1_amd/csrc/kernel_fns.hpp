@@ -54,10 +54,11 @@ constexpr KernelFn conv_fn() {
 namespace sys1 {
 // A skinny-M kernel per epilogue; null where the epilogue does not apply
 // (gated epilogues need whole 32-row gate/up groups, an even FN; RoPE half
-// or whole heads, FN = 2 or 4; the conv runs on the tile kernels).
+// or whole heads, FN = 2 or 4, the half ones up to 64 rows: 64x64 never takes
+// more tiles or bytes than 128x32; the conv runs on the tile kernels).
 template <int FM, int FN, int NW, int U, int EPI>
 constexpr KernelFn skinny_fn() {
-  if constexpr ((epi_gated(EPI) && FN % 2 != 0) || (EPI == kEpiRopeQkv && FN != 2 && FN != 4) ||
+  if constexpr ((epi_gated(EPI) && FN % 2 != 0) || (EPI == kEpiRopeQkv && FN != 4 && (FN != 2 || FM > 4)) ||
                 epi_base(EPI) == kEpiConvSilu)
     return nullptr;
   else

@@ -146,7 +146,8 @@ namespace {
 const KernelEntry kKernels[] = {
 #define SYS1_SHAPE(name, BM, BN, WM, WN, ST, BK, OCC, SK, PW, EFF, SWEFF, LKEFF) \
   KernelEntry{#name, BM, BN, (WM * WN + (PW > 0 ? PW : 0)) * 64, OCC, SK, EFF, BK, ST, BN / WN, WM, PW, SWEFF, LKEFF, sys1::name##_fns, false},
-// (skinny entries: tn 16 and wm 0 keep the RoPE and fused-conv calls off them)
+// (skinny entries: tn 16 and wm 0 keep forced RoPE and fused-conv calls off
+// them; RoPE runs on them by skinny_pick alone)
 #define SYS1_SKINNY(name, FM, FN, NW, U) \
   KernelEntry{#name, 16 * FM, 16 * FN, NW * 64, 1, false, 1.0f, 32, 0, 16, 0, 0, 0.0f, 0.0f, sys1::name##_fns, true},
 #include "shapes.def"
@@ -421,12 +422,15 @@ int64_t halo_rows(const KernelEntry& e, int64_t M, int halo) {
 constexpr int64_t kSkinnyMaxM = 4096;
 constexpr int64_t kSkinnyWeightBytes = 32 << 20;
 constexpr int64_t kSkinnyCuBytes = 704 << 10;
-// With RoPE, whose tile and stream-K plans are the head-aligned ones: up to
-// 64x64 skinny tiles won (us, against those plans: hidden 768 at 1 / 61 /
-// 300 / 400 tokens 5.5 / 6.1 / 9.1 / 9.7 against 11.7 / 19.0 / 12.4 / 12.5;
-// hidden 1024 at 16 / 300 tokens 6.5 / 11.2 against 11.2 / 14.2), 128x64
-// ones tied or lost (768 at 600: 12.9 against 12.6, 1024 at 600: 16.8
-// against 14.7).
+// With RoPE, whose tile and stream-K plans are the head-aligned ones: the
+// 64x64 skinny tiles and smaller ones won (us, against those plans: hidden 768
+// at 1 / 61 / 300 / 400 tokens 5.5 / 6.1 / 9.1 / 9.7 against 11.7 / 19.0 /
+// 12.4 / 12.5; hidden 1024 at 16 / 300 tokens 6.5 / 11.2 against 11.2 / 14.2).
+// 128x64 ones tied or lost at those widths (768 at 600: 12.9 against 12.6,
+// 1024 at 600: 16.8 against 14.7) and won below, where 192 rows of K stay
+// within the limit (K <= 682): 8 heads, K = 512 at 641 / 1025 tokens 10.7 /
+// 11.5 against 11.7 / 12.9, 10 heads, K = 640 13.0 / 14.9 against 14.6 / 14.7,
+// 8 heads, K = 256 7.5 / 8.8 against 9.1 / 9.6.
 constexpr int64_t kSkinnyRopeCuBytes = 256 << 10;
 
 // The skinny kernels address x and w through one buffer descriptor each,

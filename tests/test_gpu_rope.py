@@ -155,11 +155,13 @@ def test_rope_qkv_errors(dev):
     assert rq(x, torch.zeros(4, dtype=torch.int32, device="cuda")).shape == (3, 4, 128)
 
 
-@pytest.mark.parametrize("hidden,heads", [(768, 12), (1024, 16), (200, 1), (256, 5)])
+@pytest.mark.parametrize("hidden,heads", [(768, 12), (1024, 16), (200, 1), (256, 5), (512, 8)])
 def test_rope_qkv_of_small_batches(dev, orc, hidden, heads):
     """The skinny kernels' RoPE (half and whole heads per workgroup), over the
-    token counts whose plans are their shapes, ragged last tile rows and K
-    not a multiple of a k-step.  The elementwise bound of the file's head."""
+    token counts whose plans are each of their shapes (128x64 for 512 x 8 at
+    701, the others in all), ragged last tile rows and K not a multiple of a
+    k-step; the same bits from a column slice of x into an output that is not
+    16-byte aligned.  The elementwise bound of the file's head."""
     from sys1_amd.batching import draw_lengths, positions
     from sys1_amd.rope import RopeQkvLinear
     cos, sin = orc.rope_tables(160000.0, 64, 512)
@@ -172,6 +174,12 @@ def test_rope_qkv_of_small_batches(dev, orc, hidden, heads):
         x = orc.fill_normal((M, hidden), 20 + M)
         print(f"[gpu] rope small hidden={hidden} heads={heads} M={M}", flush=True)
         exp, proj = _expected(orc, x, w, cos, sin, pos, heads)
-        got = to_np(rq(to_gpu_bf16(x, torch), torch.from_numpy(pos).cuda()))
+        xg, pg = to_gpu_bf16(x, torch), torch.from_numpy(pos).cuda()
+        y = rq(xg, pg)
+        wide = torch.full((M, hidden + 24), float("nan"), dtype=torch.bfloat16, device="cuda:0")
+        wide[:, 8:8 + hidden] = xg
+        out = torch.empty(y.numel() + 4, dtype=torch.bfloat16, device="cuda:0")[4:].view(y.shape)
+        assert torch.equal(rq.forward_into(wide[:, 8:8 + hidden], pg, out), y)
+        got = to_np(y)
         for p in range(3):
             _check(orc, got[p], exp[p], f"M={M} plane {p}", _pair_norm(proj, p, heads) if p < 2 else None)
