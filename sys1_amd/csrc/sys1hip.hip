@@ -121,10 +121,11 @@ struct KernelEntry {
   float efficiency;     // measured MFMA efficiency of the shape, fitted to a sweep of the
                         // projection shapes (ModernBERT base/large, Qwen, square)
   int bk;               // k-tile depth
-  int stages;           // LDS pipeline stages (stages - 1 k-tiles in flight)
+  int stages;           // LDS pipeline stages (ping-pong: slots of a quarter k-tile; see in_flight)
   int tn;               // output columns per wave (the RoPE epilogue needs 64: one head)
   int wm;               // waves along M (the conv epilogue needs 1: a wave holds every row)
-  int pw;               // producer waves (0: the compute waves issue the refills)
+  int pw;               // producer waves (0: the compute waves issue the refills; -1: they
+                        // do, in the ping-pong schedule)
   float swiglu_efficiency;  // efficiency with a SwiGLU epilogue, when it differs (0: the same)
   float long_k_efficiency;  // efficiency for long K (model_cost), when it differs (0: the same)
   const KernelFn* fn;   // [kEpiCount]: the shape's kernel per epilogue (null: not built)
@@ -187,7 +188,7 @@ bool needs_stats_pass(const KernelEntry& e, int32_t norm, int64_t K) {
 //   - its compute: MFMA cycles (derated by the shape's fitted efficiency) or
 //     operand loads at kLoadBytesPerClk per CU, times the workgroups sharing
 //     the CU, and
-//   - the load latency spread over the k-tiles in flight (stages - 1).
+//   - the load latency spread over the k-tiles in flight.
 // A split tile costs its last arriving owner the arrival latency plus
 // reading every owner's f32 partial.  The call is bounded below by the
 // weight bytes at a sustained HBM rate.  The constants and efficiencies are
@@ -236,6 +237,10 @@ int occupancy(const Context* c, int id, int epi) {
 // one workgroup per CU against the plain shape at two).
 constexpr double kLowOccupancyRate = 0.7;
 
+// K-tiles requested ahead of the one multiplied: every stage but its own, or
+// for the ping-pong ring every slot but the one read, four to a k-tile.
+double in_flight(const KernelEntry& e) { return e.pw < 0 ? (e.stages - 1) / 4.0 : e.stages - 1; }
+
 // (*busy: the same without the HBM floor.)
 double model_cost(const Context* c, int id, int epi, int64_t M, int64_t N, int64_t K,
                   int64_t grid, int64_t dp, double* busy) {
@@ -259,14 +264,13 @@ double model_cost(const Context* c, int id, int epi, int64_t M, int64_t N, int64
   // the CU count), is priced the same way: measured ~2160 cycles per k-tile
   // for the 128x128 producer-wave shape on 256 tiles of 1024x2624.
   const bool lone_pair = occupancy(c, id, epi) >= 2 && grid <= c->cus;
-  const double latency = e.pw && grid >= c->cus && !lone_pair ? kProducerLatencyClk : kLatencyClk;
-  const double per_kt = std::max(share * std::max(mfma, load), latency / (e.stages - 1));
+  const double latency = e.pw > 0 && grid >= c->cus && !lone_pair ? kProducerLatencyClk : kLatencyClk;
+  const double per_kt = std::max(share * std::max(mfma, load), latency / in_flight(e));
   // (A bias that the tile epilogue has no registers to read in a batch -- its
   // rule: accumulators and bias vectors above half of a wave's registers --
-  // costs half as much again, none of it
-  // hidden by a second workgroup: vision qkv at 8192 / 16384 rows ran 77 / 161 us
-  // on the 256x160 and 128x128 plans, 67 / 133 on the ping-pong shape, which
-  // batches it.)
+  // costs half as much again, none of it hidden by a second workgroup: vision
+  // qkv at 8192 / 16384 rows ran 77 / 161 us on the 256x160 and 128x128 plans,
+  // 67 / 133 on the ping-pong shape, which batches it.)
   const int waves_per_simd = (e.threads / 64 * e.occupancy + 3) / 4;
   const int fn = e.tn / 32, blocks = e.streamk ? 0 : e.bm / e.wm / 32 * fn;
   const bool bias = epi == kEpiBias || epi == kEpiBiasGelu || epi == kEpiBiasResidual || epi == kEpiBiasGeluTanh;
@@ -511,11 +515,11 @@ Plan price_plans(const Context* c, int64_t M0, int64_t N, int64_t K, bool wide, 
       // split tile to fix up (measured: Qwen3.5-27B gate_up at M = 128,
       // 182 tiles of 128x192, 76.0 us against 81.6-84.1 us on the stream-K
       // hybrid whose 16 split tiles are summed after the stream).
-      if (e.pw < 0 && M <= kPingPongMinM) continue;
       const int64_t whole = cdiv(M, e.bm) * cdiv(N, e.bn);
       if (!e.streamk && M <= 128 &&
           !(M > 64 && cdiv(M, e.bm) == 1 && whole <= (int64_t)c->cus && 3 * whole >= 2 * (int64_t)c->cus))
         continue;
+      if (e.pw < 0 && M <= kPingPongMinM) continue;
     }
     const int64_t gmax = max_grid(c, id, epi, M, N, K);
     if (c->forced_grid > 0) {

@@ -81,6 +81,15 @@ E = _lib
     (256, 2048, 6144, E.EPI_RESIDUAL, "stream_32x256_s4_w1x4_p4_g256"),
     (576, 2048, 6144, E.EPI_RESIDUAL, "stream_128x128_s4_w2x2_p4_g256"),
     (960, 2048, 4096, E.EPI_RESIDUAL, "stream_128x128_s4_w2x2_p4_g256"),
+    # two tile plans at the weight stream's floor: the one with less work
+    (200, 34816, 5120, E.EPI_SWIGLU, "tile_256x160_s3_w8x1_p4_g218"),
+    (256, 34816, 5120, E.EPI_SWIGLU, "tile_256x160_s3_w8x1_p4_g218"),
+    # the ping-pong shape: above 640 tokens, long K, and a bias that 256x160
+    # and 128x128 tiles have no registers to batch
+    (640, 16480, 5120, E.EPI_NONE, "tile_128x192_s3_w4x2_p4_g256"),
+    (768, 16480, 5120, E.EPI_NONE, "tile_256x256_s10_w2x4_pp_g195"),
+    (4096, 34816, 5120, E.EPI_SWIGLU, "tile_256x256_s10_w2x4_pp_g256"),
+    (8192, 3456, 1152, E.EPI_BIAS, "tile_256x256_s10_w2x4_pp_g256"),
 ])
 def test_plans_of_the_measured_workloads(M, N, K, epi, plan):
     kid, grid, name = _lib.plan_kernel(M, N, K, epi)
