@@ -1251,9 +1251,12 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) /
       freed = slot;
       slot = slot + 1 == SLOTS ? 0 : slot + 1;
     };
+    const bool second = wave >= S::kWaves / 2;  // the group half a phase behind
     // One phase of unit type T: its fragments, a request into the slot the
     // last phase freed, the wait for the next phase's unit; the barrier; the
-    // quadrant that the fragments complete; the barrier.
+    // quadrant that the fragments complete; the barrier.  (Not the second
+    // group's last one, which would have the first group's last epilogue in
+    // front of its own; each group then passes as many.)
     auto phase = [&](auto tc, bool load, bool mul) {
       constexpr int T = decltype(tc)::value;
       if (load) {
@@ -1278,7 +1281,7 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) /
       }
       if (load) advance(std::integral_constant<int, (T + kAhead) % 4>());
       __builtin_amdgcn_s_setprio(0);
-      bar();
+      if (load || !second) bar();
     };
     using std::integral_constant;
     // Prologue: the first kAhead units, the first of them landed.
@@ -1292,7 +1295,6 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) /
     }
     vm_wait<kInFlight>();
     bar();
-    const bool second = wave >= S::kWaves / 2;  // the group half a phase behind
     if (second) bar();
     Segment csg = walk.first_segment();
     int ckt = csg.kt0;
@@ -1310,7 +1312,6 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) /
     }
     phase(integral_constant<int, 0>(), false, true);
     epilogue(walk.row0(csg.tm), csg.tn * BN, 0);
-    if (!second) bar();
     vm_wait<0>();  // the zero-size refills of the last units write LDS too
     return;
   }

@@ -578,6 +578,7 @@ def test_blocked_weight_layout_is_bitwise_row_major(dev, orc):
 @pytest.mark.parametrize("M,N,K,grid", [
     (1, 8, 8, 0), (256, 256, 64, 0), (257, 264, 72, 0), (511, 520, 128, 1), (700, 800, 200, 2),
     (1030, 520, 1032, 3), (513, 1284, 640, 5),
+    (1030, 1300, 64, 3), (700, 1284, 40, 2), (1600, 800, 8, 1),  # one k-tile a tile: requests two tiles ahead
 ])
 @pytest.mark.parametrize("blocked", [False, True])
 def test_ping_pong_tiles_at_their_edges(dev, orc, M, N, K, grid, blocked):
