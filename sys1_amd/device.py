@@ -14,9 +14,6 @@ import torch
 from . import _lib
 
 
-_raw_stream = torch._C._cuda_getCurrentRawStream
-
-
 class HipDevice:
     def __init__(self, index: int = 0):
         L = _lib.load()
@@ -27,6 +24,8 @@ class HipDevice:
         self.index = int(index)
         self.torch_device = torch.device("cuda", self.index)
         self._stream = None
+        # (looked up here: a CPU-only torch lacks it, and this module imports there)
+        self._raw_stream = torch._C._cuda_getCurrentRawStream
         torch.cuda.init()  # (the raw stream getter does not)
         self.follow_torch_stream()
 
@@ -34,7 +33,7 @@ class HipDevice:
         """Point the context at torch's current stream on this device."""
         # (torch's raw stream getter: the Stream object that current_stream
         # builds costs ~1.5 us, a fifth of a small call)
-        s = _raw_stream(self.index)
+        s = self._raw_stream(self.index)
         if s != self._stream:
             _lib.check(self._L.sys1hip_set_stream(self.ctx, ctypes.c_void_p(s)), self.ctx)
             self._stream = s

@@ -4,6 +4,8 @@ codes before touching a device (so these run without a GPU)."""
 import ctypes
 import os
 import re
+import subprocess
+import sys
 
 import pytest
 
@@ -70,6 +72,14 @@ def test_init_without_device_fails_loudly():
     assert b"no HIP device" in L.sys1hip_last_error(None)
     with pytest.raises(_lib.Sys1HipError):
         _lib.check(rc)
+
+
+def test_modules_import_under_a_cpu_only_torch():
+    # (such a torch has no raw stream getter; in a process of its own, so that
+    # no module is loaded already)
+    code = ("import torch; del torch._C._cuda_getCurrentRawStream; "
+            "import sys1_amd.device, sys1_amd.linear, sys1_amd.norm, sys1_amd.rope, sys1_amd.deltanet, sys1_amd.stacks")
+    subprocess.run([sys.executable, "-c", code], cwd=ROOT, check=True, timeout=300)
 
 
 # Argument validation runs before the context is dereferenced, so a dummy
