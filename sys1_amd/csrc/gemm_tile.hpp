@@ -723,7 +723,12 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) /
       conv_epilogue(m0, n0, skip);
       return;
     }
-    const int h = fk;
+    // (opaque, so that no address formed of them is kept, or spilled, across
+    // the k-loop: on the 256x160 tiles with bias and GELU it reloaded up to
+    // four a k-tile, 5% of 4096 x 4999 x 3200; the gated epilogues, of few
+    // addresses, spill more this way)
+    int row = frow, h = fk;
+    if constexpr (!epi_gated(E)) asm volatile("" : "+v"(row), "+v"(h));
     const int out_n0 = epi_gated(E) ? (n0 + wn * S::TN) / 2 : n0 + wn * S::TN;
     // Outputs, residuals and biases of calls whose rows are all 16-byte
     // aligned and within 2 GiB move by buffer instructions: a 32-bit row
@@ -779,7 +784,7 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) /
       if (!(kResLds && res_in_lds)) {
 #pragma unroll
         for (int j = 0; j < S::FM; ++j) {
-          const int m = m0 + wm * S::TM + j * 32 + frow;
+          const int m = m0 + wm * S::TM + j * 32 + row;
 #pragma unroll
           for (int i = 0; i < S::FN; ++i)
 #pragma unroll
@@ -815,7 +820,7 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) /
     constexpr bool kPipe = kWavesPerSimd <= 2 && !epi_gated(E) && E != kEpiRopeQkv &&
                            ((epi_has_bias<E>() && !kBiasRegs) || (epi_has_resid<E>() && !kResRegs));
     auto block = [&](int j, int i, const bf16x8* cbias, const bf16x8* cres) {
-      const int m = m0 + wm * S::TM + j * 32 + frow;
+      const int m = m0 + wm * S::TM + j * 32 + row;
       const bool row_ok = m < a.M;
       if constexpr (E == kEpiRopeQkv) {
         // Blocks i (even) and i+1 are the two halves of one 64-wide head
@@ -915,7 +920,7 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) /
     if constexpr (!kVec) {
 #pragma unroll
       for (int j = 0; j < S::FM; ++j) {
-        const int m = m0 + wm * S::TM + j * 32 + frow;
+        const int m = m0 + wm * S::TM + j * 32 + row;
         const bool row_ok = m < a.M;
 #pragma unroll
         for (int i = 0; i < S::FN; ++i)
@@ -969,7 +974,7 @@ __attribute__((amdgpu_waves_per_eu(((WM * WN + producer_waves(PW_)) * OCC + 3) /
           if constexpr (epi_has_resid<E>() && !kResRegs)
             if (!(kResLds && res_in_lds))  // (block() takes it from the LDS copy)
 #pragma unroll
-              for (int j = 0; j < S::FM; ++j) cres[j][gp] = get_resid(m0 + wm * S::TM + j * 32 + frow, n);
+              for (int j = 0; j < S::FM; ++j) cres[j][gp] = get_resid(m0 + wm * S::TM + j * 32 + row, n);
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
